@@ -379,7 +379,7 @@ int lu_preconditioner(int n, const double *dA, long lda, double *lu64, int64_t *
     float *a32 = (float *)c.scratch_ir;
     if ((rc = scirs_d2s(n, n, dA, lda, a32, ld32, s))) return rc;
     if ((rc = c.reset_flags(s))) return rc;
-    const bool tslu = c.work.tslu != 0;
+    const bool tslu = c.work.tslu != 0 && n > scirs_sub_max_rows<float>();
     const int kb = tslu ? c.kb_f32 : c.lu_kb<float>(n);
     const int saved = c.work.lowp_mode;
     c.work.lowp_mode = SCIRS_LOWP_BF16X6;

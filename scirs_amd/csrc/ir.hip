@@ -548,8 +548,10 @@ int gesv_ir_device(int n, int nrhs, const double *dA, long lda, const double *dB
     float *dinv_u = (float *)take(dinv_elems * sizeof(float));
     float *dmt_l = (float *)take(3 * dinv_elems * sizeof(float));   // couplings one to three blocks back
     float *dmt_u = (float *)take(3 * dinv_elems * sizeof(float));
-    const bool tslu = c.work.tslu != 0;
-    st.kb = tslu ? c.kb_f32 : c.lu_kb<float>(n);
+    // tournament pivoting only for panels of more rows than the register panel holds
+    const bool tslu = c.work.tslu != 0 && n > scirs_sub_max_rows<float>();
+    // (the narrow panels update in FP32: only where the mode's own update is as accurate)
+    st.kb = lowp == SCIRS_LOWP_FP32 || lowp == SCIRS_LOWP_BF16X6 ? c.lu_kb<float>(n) : c.kb_f32;
 
     scirs::CallEvents ev;
     if (int erc = ev.create(3)) return erc;

@@ -55,7 +55,35 @@ struct ScirsWork {
     float *tp_stage;           // 64 x SCIRS_KB_MAX rows displaced from the sub-panel's top positions
     int *tp_vlist;             // [64 + 1] positions the displaced rows move to, then their count
     int *tp_map;               // [2 * TSLU_MAP] (position, original row) of the panel's moved rows, then a count
+    // sub-panel factorisation (subpanel.hip)
+    unsigned long long *sub_key;   // [2][SCIRS_SUB_AGENTS][2] candidates (sequence-tagged words)
+    unsigned long long *sub_row;   // [2][SCIRS_SUB_AGENTS][SCIRS_SUB_W][2] their rows
+    int *sub_ctl;                  // [SCIRS_SUB_MAX][SCIRS_SUB_CTL] election of the die, count of moved rows
+    int *sub_pairs;                // [SCIRS_SUB_MAX][SCIRS_SUB_PAIRS][2] moved rows of a sub-panel
+    int *sub_arrive;               // [SCIRS_SUB_STRIPS] arrival counts (zero between launches)
+    int *sub_label;                // [SCIRS_SUB_ROWS] the identity between launches
 };
+
+// Sub-panel width, waves of its exchange, moved rows at most, sub-panels per
+// factorisation, control words of one (8 dies' counts 32 apart, the elected die,
+// the moved-row count), strips of a sub-panel update, rows of the matrix.
+enum { SCIRS_SUB_W = 32, SCIRS_SUB_AGENTS = 128, SCIRS_SUB_PAIRS = 64, SCIRS_SUB_MAX = 2048, SCIRS_SUB_CTL = 320,
+       SCIRS_SUB_COUNT = 288, SCIRS_SUB_STRIPS = 2048, SCIRS_SUB_ROWS = 1 << 16 };
+
+// Factor columns c0 .. c0 + w - 1 (w <= 32), rows c0 .. rows - 1, with partial
+// pivoting; the rows that move (destination, source) go to pairs, their number is
+// added to *npairs.  elect: SCIRS_SUB_COUNT zeroed words.
+template <typename T>
+int scirs_sub_panel(T *A, long lda, int rows, int c0, int w, int *pairs, int *npairs, int *elect, ScirsWork &wk,
+                    hipStream_t s);
+template <typename T> int scirs_sub_max_rows();
+// That sub-panel's interchanges, U12 = L11^-1 A12 and the update of columns
+// [ca, cb), its interchanges on columns [la, lb), and, ncomp > 0, the composition
+// of the ncomp lists at cpairs / cn (SCIRS_SUB_CTL counts apart) into one.
+template <typename T>
+int scirs_sub_apply(T *A, long lda, int rows, int c0, int w, int ca, int cb, int la, int lb, const int *pairs,
+                    const int *npairs, int ncomp, const int *cpairs, const int *cn, int *out_pairs, int *out_n,
+                    ScirsWork &wk, hipStream_t s);
 
 enum { TSLU_MAXLEV = 6, TSLU_MAXNODE = 512, TSLU_MAP = 512 };
 
@@ -156,9 +184,8 @@ int scirs_getrf_device(int m, int n, T *A, long lda, int kb, ScirsWork &w, hipSt
 template <typename T>
 int scirs_transpose_lower(int n, const T *L, long ldl, T *U, long ldu, hipStream_t s);
 
-// Panel width for an m-row factorisation: the widest of kb, 64, 32 (never above
-// kb) at which all m rows of a panel fit one workgroup's LDS, so every panel is
-// factored by one workgroup without inter-workgroup exchange; kb when none fits.
+// Panel width for an m-row factorisation: 32 while single sub-panels with an
+// update of every column beat kb-wide panels with look-ahead, else kb.
 int scirs_lu_panel_kb(int m, int kb, size_t elem_bytes);
 
 // Row permutation produced by the last getrf: perm[i] = original row now at i
