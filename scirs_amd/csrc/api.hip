@@ -147,8 +147,7 @@ int Context::init(int dev)
                  xrj_b = rep * 2 * (size_t)kbmax * 2 * 8, flags_b = 64 * sizeof(int),
                  pairs_b = (size_t)work.max_panels * 4 * kbmax * sizeof(int),
                  npairs_b = (size_t)work.max_panels * sizeof(int),
-                 linv_b = 2 * 128 * 128 * sizeof(float),   // two FP32 L11^-1 (double-buffered)
-                 linv64_b = 128 * 128 * sizeof(double);
+                 linv_b = 2 * 128 * 128 * sizeof(float);   // two FP32 L11^-1 (double-buffered)
     const size_t tpc_b = (size_t)TSLU_MAXLEV * TSLU_MAXNODE * 65 * 8, tpn_b = (size_t)TSLU_MAXLEV * TSLU_MAXNODE * 4,
                  tpu_b = 64 * 64 * sizeof(float), tpr_b = 64 * 64 * sizeof(float),
                  tpt_b = 64 * (size_t)kbmax * sizeof(float), tpv_b = 65 * sizeof(int),
@@ -157,7 +156,7 @@ int Context::init(int dev)
                  sc_b = (size_t)SCIRS_SUB_MAX * SCIRS_SUB_CTL * 4, sp_b = (size_t)SCIRS_SUB_MAX * SCIRS_SUB_PAIRS * 2 * 4,
                  sa_b = (size_t)SCIRS_SUB_STRIPS * 4, sl_b = (size_t)SCIRS_SUB_ROWS * 4;
     for (size_t b : {sk_b, sr_b, sc_b, sp_b, sa_b, sl_b}) bytes += (b + 255) & ~(size_t)255;
-    for (size_t b : {xw_b, xrow_b, xrj_b, flags_b, pairs_b, npairs_b, linv_b, linv64_b, tpc_b, tpn_b, tpu_b, tpr_b, tpt_b, tpt_b,
+    for (size_t b : {xw_b, xrow_b, xrj_b, flags_b, pairs_b, npairs_b, linv_b, tpc_b, tpn_b, tpu_b, tpr_b, tpt_b, tpt_b,
                      tpv_b, tpm_b})
         bytes += (b + 255) & ~(size_t)255;
     char *base = nullptr;
@@ -179,7 +178,6 @@ int Context::init(int dev)
     work.pairs = (int *)take(pairs_b);
     work.npairs = (int *)take(npairs_b);
     work.linv = take(linv_b);
-    work.linv64 = (double *)take(linv64_b);
     work.tp_cand = (unsigned long long *)take(tpc_b);
     work.tp_cnt = (int *)take(tpn_b);
     work.tp_uinv = (float *)take(tpu_b);

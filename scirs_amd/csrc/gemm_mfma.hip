@@ -12,6 +12,7 @@
 // and B columns in that XCD's L2: hardware dispatches workgroup w to XCD w % 8.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "lanes.hpp"
 #include "tile_map.hpp"
 #include <cstdlib>
 
@@ -194,11 +195,7 @@ __global__ __launch_bounds__(NTHREADS, CPRE ? 1 : 2) void gemm_sub_kernel(GemmAr
 // work instead of preceding it (the memory counter retires loads in order: a
 // wait for the slab operands never waits for C).  Operands come in as 16-byte
 // loads; B goes to LDS as 16-byte stores.
-// ASSIGN: C = A op(B) instead (C is not read; A enters LDS unnegated): the
-// Cholesky TRSM L21 = A21 L11^-T, in place — a workgroup reads all K columns of
-// its rows before it writes them, and with N <= 128 no other workgroup reads
-// those rows.
-template <int KS, bool VEC, int OCC, bool TRANS_B, bool ASSIGN = false>
+template <int KS, bool VEC, int OCC, bool TRANS_B>
 __global__ __launch_bounds__(NTHREADS, OCC) void dgemm_fold_kernel(GemmArgs<double> g)
 {
     static_assert(KS >= 8 && KS % 8 == 0, "eight half block rows of C folded over the slabs");
@@ -258,7 +255,7 @@ __global__ __launch_bounds__(NTHREADS, OCC) void dgemm_fold_kernel(GemmArgs<doub
     };
     auto store_slab = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) As[buf][(a_k + i) * LDA_S + a_r] = ASSIGN ? ra[i] : -ra[i];
+        for (int i = 0; i < 8; ++i) As[buf][(a_k + i) * LDA_S + a_r] = -ra[i];
         if (TRANS_B) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) Bs[buf][(a_k + i) * LDB_S + a_r] = rb[i];
@@ -310,10 +307,8 @@ __global__ __launch_bounds__(NTHREADS, OCC) void dgemm_fold_kernel(GemmArgs<doub
         if (s + 1 < KS) load_slab((s + 1) * BK);
         // C half row h: loaded during slab h * KS / 8, folded in the next slab
         constexpr int STEP = KS / 8;
-        if (!ASSIGN) {
-            if (s >= STEP && s % STEP == 0) fold_c(s / STEP - 1);
-            if (s % STEP == 0) load_c(s / STEP);
-        }
+        if (s >= STEP && s % STEP == 0) fold_c(s / STEP - 1);
+        if (s % STEP == 0) load_c(s / STEP);
         // keep the loads ahead of the matrix-core work and the LDS stores behind it
         __builtin_amdgcn_sched_barrier(0);
         const double *as = As[buf];
@@ -337,8 +332,8 @@ __global__ __launch_bounds__(NTHREADS, OCC) void dgemm_fold_kernel(GemmArgs<doub
         if (s + 1 < KS) store_slab(buf ^ 1);
         __syncthreads();
     }
-    if (!ASSIGN) fold_c(7);
-    // epilogue: C = C - A B (or A B), already in the accumulators
+    fold_c(7);
+    // epilogue: C = C - A B, already in the accumulators
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
@@ -354,6 +349,78 @@ __global__ __launch_bounds__(NTHREADS, OCC) void dgemm_fold_kernel(GemmArgs<doub
     }
 }
 
+// C (M x N) -= A B^T with K = 128 in 64 x 64 tiles, operands straight from L2 into the
+// matrix-core layout: small updates, whose 128 x 128 tiles would leave most CUs idle
+// and take 27 us a tile (8 us a tile here; the large tiles reuse their operands twice
+// as often and win once they fill the device).  lower: only tiles that touch C's lower
+// triangle.  k-order as above.
+struct Syrk64Args {
+    const double *A, *B; double *C;
+    long lda, ldb, ldc;
+    int M, N, lower;
+    const int *info;
+};
+__global__ __launch_bounds__(NTHREADS) void gemm_nt64_kernel(Syrk64Args g)
+{
+    if (*g.info != 0) return;
+    using lanes::Mf;
+    typedef lanes::Vec16u<double>::type Vu;
+    const int row0 = 64 * blockIdx.y, col0 = 64 * blockIdx.x;
+    if (g.lower && col0 > row0 + 63) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int l16 = lane & 15, grp = lane >> 4, r0 = row0 + 32 * (wave >> 1), c0 = col0 + 32 * (wave & 1);
+    if (r0 >= g.M || c0 >= g.N) return;
+    const double *pa[2], *pb[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        pa[i] = g.A + (long)min(r0 + 16 * i + l16, g.M - 1) * g.lda + 8 * grp;
+        pb[i] = g.B + (long)min(c0 + 16 * i + l16, g.N - 1) * g.ldb + 8 * grp;
+    }
+    double fa[2][2][8], fb[2][2][8];
+    auto load = [&](int k, double (&x)[2][8], double (&y)[2][8]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const Vu u = *reinterpret_cast<const Vu *>(pa[i] + 32 * k + e);
+                const Vu v = *reinterpret_cast<const Vu *>(pb[i] + 32 * k + e);
+                x[i][e] = -u[0]; x[i][e + 1] = -u[1];
+                y[i][e] = v[0]; y[i][e + 1] = v[1];
+            }
+    };
+    Mf<double>::V acc[2][2];
+    load(0, fa[0], fb[0]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                acc[i][j][q] = g.C[(long)min(r0 + 16 * i + Mf<double>::row(grp, q), g.M - 1) * g.ldc +
+                                   min(c0 + 16 * j + l16, g.N - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (k < 3) load(k + 1, fa[(k + 1) & 1], fb[(k + 1) & 1]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = Mf<double>::mac(fa[k & 1][i][e], fb[k & 1][j][e], acc[i][j]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = r0 + 16 * i + Mf<double>::row(grp, q);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int c = c0 + 16 * j + l16;
+                if (r < g.M && c < g.N) g.C[(long)r * g.ldc + c] = acc[i][j][q];
+            }
+        }
+}
+
 template <typename T>
 int launch_gemm_sub(int M, int N, int K, const T *A, long lda, const T *B, long ldb, int trans_b, T *C,
                     long ldc, int lower, const int *info, hipStream_t stream)
@@ -366,6 +433,17 @@ int launch_gemm_sub(int M, int N, int K, const T *A, long lda, const T *B, long 
     g.tiles_n = (N + BN - 1) / BN;
     g.lower = lower;
     g.info = info;
+    if constexpr (sizeof(T) == 8) {
+        // while 128 x 128 tiles would leave half the CUs idle (n = 1000 Cholesky solve 885
+        // against 1011 us with large tiles only, 899 us with this form up to 400 tiles)
+        const int tiles = lower ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * g.tiles_n;
+        if (trans_b && K == 8 * BK && info && tiles <= 128) {
+            Syrk64Args a{A, B, C, lda, ldb, ldc, M, N, lower, info};
+            hipLaunchKernelGGL(gemm_nt64_kernel, dim3((N + 63) / 64, (M + 63) / 64), dim3(NTHREADS), 0, stream, a);
+            SCIRS_HIP_CHECK(hipGetLastError());
+            return SCIRS_OK;
+        }
+    }
     const int nwg = (g.tiles_m * g.tiles_n + 7) / 8 * 8;
     // FP64: C prefetched at one workgroup per CU by default, which also leaves
     // room on each CU for the look-ahead panel running beside the update
@@ -412,31 +490,6 @@ int scirs_launch_dgemm_sub(int M, int N, int K, const double *A, long lda, const
                            hipStream_t stream)
 {
     return launch_gemm_sub<double>(M, N, K, A, lda, B, ldb, trans_b, C, ldc, lower, info, stream);
-}
-
-int scirs_launch_dgemm_assign_t(int M, int N, int K, const double *A, long lda, const double *B, long ldb,
-                                double *C, long ldc, const int *info, hipStream_t stream)
-{
-    if (M <= 0 || N <= 0) return SCIRS_OK;
-    if (K != 8 * BK || N > BN) {
-        scirs_set_error("dgemm_assign_t: K must be %d and N at most %d (got K=%d N=%d)", 8 * BK, BN, K, N);
-        return SCIRS_ERR_ARG;
-    }
-    GemmArgs<double> g;
-    g.M = M; g.N = N; g.K = K;
-    g.A = A; g.lda = lda; g.B = B; g.ldb = ldb; g.C = C; g.ldc = ldc;
-    g.tiles_m = (M + BM - 1) / BM;
-    g.tiles_n = 1;
-    g.lower = 0;
-    g.info = info;
-    const int nwg = (g.tiles_m + 7) / 8 * 8;
-    const bool vec = ((uintptr_t)A % 16 == 0) && ((uintptr_t)B % 16 == 0) && lda % 2 == 0 && ldb % 2 == 0;
-    if (vec)
-        hipLaunchKernelGGL((dgemm_fold_kernel<8, true, 2, true, true>), dim3(nwg), dim3(NTHREADS), 0, stream, g);
-    else
-        hipLaunchKernelGGL((dgemm_fold_kernel<8, false, 1, true, true>), dim3(nwg), dim3(NTHREADS), 0, stream, g);
-    SCIRS_HIP_CHECK(hipGetLastError());
-    return SCIRS_OK;
 }
 
 int scirs_launch_sgemm_f32_sub(int M, int N, int K, const float *A, long lda, const float *B, long ldb,

@@ -2,13 +2,13 @@
 // Only the lower triangle of A is read, as in scirs2-linalg/src/lapack.rs:632-679,
 // and the strict upper triangle of the result is zeroed so the output is the
 // reference's L.  Per block of kb columns at k0:
-//   1. potf2 — one workgroup factors the kb x kb diagonal block in LDS; the
-//      reference's test `a_ii - sum <= 0` (lapack.rs:661-670) sets
+//   1. chol_panel — the diagonal block's factor and L21 = A21 L11^-T in one
+//      launch; the reference's test `a_ii - sum <= 0` (lapack.rs:661-670) sets
 //      info = row + 1 and stops.
-//   2. trsm  — L21 = A21 L11^-T, 64 rows per workgroup, L11 packed in LDS.
-//   3. syrk  — A22 -= L21 L21^T on the matrix cores (lower tiles only).
+//   2. syrk — A22 -= L21 L21^T on the matrix cores (lower tiles only).
 #include "common.hpp"
 #include "kernels.hpp"
+#include "lanes.hpp"
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -32,361 +32,285 @@ __device__ __forceinline__ double readlane_t<double>(double v, int k)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-__device__ __forceinline__ void wave_sync()
+// A panel of kb <= 128 columns in one launch: the diagonal block's factor and the
+// rows below, L21 = A21 L11^-T by substitution (lapack.rs:661-676: sqrt, true
+// division).  Every workgroup factors the diagonal block for itself — 32 columns at a
+// time, and a wave needs nothing from another while it does: its lanes 0..31 hold the
+// 32 diagonal rows (the same in all waves), lanes 32..63 the rows it is responsible
+// for, groups 1..3 of the diagonal block (waves 0..2) and 32 rows of A21 (wave 3).
+// Column j: the diagonal by readlane, its square root and reciprocal, l = a / sqrt
+// (one residual correction: correctly rounded), and a_c -= l l_c with l_c handed to all
+// lanes by two permlane swaps and DPP (lanes.hpp).  Between the 32-column steps the
+// waves exchange their L through LDS and update their later columns, which wait in
+// registers in the matrix-core layout.  The last workgroup to have read the diagonal
+// block (an arrival count, nobody waits) writes it back.
+// Bound by the column chain (about 400 cycles a column).  Measured for one 128-column
+// panel: 36 us whatever the rows below (up to one workgroup per CU), against
+// 78 (diagonal block) + 36 (its inverse) + 23 us (product) in three launches before.
+// One a_jj - sum <= 0 sets info = row + 1 and stops.
+template <typename T> struct CholPanelArgs {
+    T *A; long lda;
+    int k0, kb, n;
+    int *arrive;      // zero between launches
+    int *info; double *info_val;
+};
+// x's lanes 0..15 (lo) and 16..31 (hi) in every row of 16 lanes
+__device__ __forceinline__ void spread(unsigned x, unsigned &lo, unsigned &hi)
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    lo = __builtin_amdgcn_permlane32_swap(p[0], p[0], false, false)[0];
+    hi = __builtin_amdgcn_permlane32_swap(p[1], p[1], false, false)[0];
+}
+__device__ __forceinline__ void spread(double x, double (&pr)[2])
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    unsigned l0, l1, h0, h1;
+    spread((unsigned)b, l0, l1);
+    spread((unsigned)(b >> 32), h0, h1);
+    pr[0] = __longlong_as_double((long long)(((unsigned long long)h0 << 32) | l0));
+    pr[1] = __longlong_as_double((long long)(((unsigned long long)h1 << 32) | l1));
+}
+__device__ __forceinline__ void spread(float x, float (&pr)[2])
+{
+    unsigned l0, l1;
+    spread(__float_as_uint(x), l0, l1);
+    pr[0] = __uint_as_float(l0);
+    pr[1] = __uint_as_float(l1);
+}
+// 1/p to an ulp, and a/p from it by residual corrections
+__device__ __forceinline__ double recip(double p)
+{
+    double r = __builtin_amdgcn_rcp(p);
+    r = fma(r, fma(-p, r, 1.0), r);
+    return fma(r, fma(-p, r, 1.0), r);
+}
+__device__ __forceinline__ float recip(float p)
+{
+    const float r = __builtin_amdgcn_rcpf(p);
+    return fmaf(r, fmaf(-p, r, 1.0f), r);
+}
+__device__ __forceinline__ double quot(double a, double p, double r)
+{
+    const double q = a * r;
+    return fma(fma(-q, p, a), r, q);
+}
+__device__ __forceinline__ float quot(float a, float p, float r)
+{
+    float q = a * r;
+    q = fmaf(fmaf(-q, p, a), r, q);
+    return fmaf(fmaf(-q, p, a), r, q);
 }
 
-typedef double dv4 __attribute__((ext_vector_type(4)));
-typedef float fv4 __attribute__((ext_vector_type(4)));
-template <typename T> struct MV;
-template <> struct MV<double> {
-    typedef dv4 V;
-    static __device__ __forceinline__ V mfma(double a, double b, V c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    // row of accumulator register q in lane group lk (column = lane % 16)
-    static __device__ __forceinline__ int row(int lk, int q) { return lk + 4 * q; }
-};
-template <> struct MV<float> {
-    typedef fv4 V;
-    static __device__ __forceinline__ V mfma(float a, float b, V c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int lk, int q) { return 4 * lk + q; }
-};
-
-// The kb x kb diagonal block (kb <= 128) in LDS (lower triangle packed by
-// rows), factored in column blocks of PB = 32:
-//   A. wave 0 factors the PB x PB diagonal block, lane i holding row i in
-//      registers: per column the diagonal by readlane, sqrt, true division of
-//      the rows below (lapack.rs:661-676), the column handed to every lane
-//      through LDS, and the later columns updated — one wave, no barrier;
-//   B. the rows below solve x L_jj^T = a (one thread per row, left-looking,
-//      true division, the diagonal block read from LDS as broadcasts);
-//   C. the trailing lower triangle takes the rank-PB update on the matrix
-//      cores (16 x 16 tiles, one wave per tile).
-// The test of the reference, a_jj - sum <= 0 (lapack.rs:661-670), sets
-// info = row + 1 and stops.
-template <typename T>
-__global__ __launch_bounds__(NT) void potf2_kernel(T *A, long lda, int k0, int kb, int *info, double *info_val)
+constexpr int CP_B = 32;   // columns of a step
+// column J of the step; returns false when the diagonal is not positive
+template <typename T, int J> __device__ __forceinline__ bool chol_column(T (&a)[CP_B], T &dv)
 {
-    if (*info != 0) return;
-    constexpr int PB = 32;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    // the lower triangle, packed by rows (row r at r (r + 1) / 2): half the LDS
-    // of a square tile, so the kernel fits on a CU beside one workgroup of the
-    // trailing update running on the other stream
-    T *S = reinterpret_cast<T *>(smem_raw);
-    auto pk = [](int r, int c) { return r * (r + 1) / 2 + c; };
-    __shared__ T colb[2][PB];
-    // the factored diagonal block, unpacked, so that phase B addresses it with
-    // one base register and constant offsets
-    __shared__ T Dsq[PB][PB + 1];
-    __shared__ int s_fail;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    T *D = A + (long)k0 * lda + k0;
-    // rows wave, wave + 4, ...: 64 loads in flight per lane before any
-    // LDS store (a load-then-store loop would wait for each row in turn)
-    for (int i0 = wave; i0 < kb; i0 += 32 * (NT / 64)) {
-        T v[32][2];
+    dv = readlane_t<T>(a[J], J);
+    if (__builtin_expect(!(dv > (T)0), 0)) return false;
+    const T s = sqrt(dv), r = recip(s);   // (a root is neither tiny nor huge: no scaling)
+    T q = quot(a[J], s, r);
+    if (__builtin_expect(dv > (T)(sizeof(T) == 8 ? DBL_MAX : FLT_MAX), 0)) q = a[J] / s;   // infinite: no residual
+    const T l = (threadIdx.x & 63) == J ? s : q;
+    a[J] = l;
+    T pr[2];
+    spread(l, pr);
+    constexpr int c0 = J + 1;
+    if constexpr (c0 < CP_B) {
+        // up to the next multiple of eight, then whole blocks
+        constexpr int n0 = (8 - (c0 & 7)) & 7;
+        if constexpr (n0 > 0) lanes::fmac_row<c0 & 15, n0 ? n0 : 1>(&a[c0], pr[c0 >> 4], l);
+        constexpr int b0 = (c0 + 7) / 8;
+        if constexpr (b0 < 1) lanes::fmac_row<0, 8>(&a[0], pr[0], l);
+        if constexpr (b0 < 2) lanes::fmac_row<8, 8>(&a[8], pr[0], l);
+        if constexpr (b0 < 3) lanes::fmac_row<0, 8>(&a[16], pr[1], l);
+        if constexpr (b0 < 4) lanes::fmac_row<8, 8>(&a[24], pr[1], l);
+    }
+    return true;
+}
+// columns J .. 31; the failing column, or -1
+template <typename T, int J> __device__ __forceinline__ int chol_columns(T (&a)[CP_B], T &dv)
+{
+    if constexpr (J < CP_B) {
+        if (!chol_column<T, J>(a, dv)) return J;
+        return chol_columns<T, J + 1>(a, dv);
+    } else {
+        return -1;
+    }
+}
+
+template <typename T> __global__ __launch_bounds__(NT, 2) void chol_panel_kernel(CholPanelArgs<T> g)
+{
+    if (*g.info != 0) return;
+    using lanes::Mf;
+    typedef typename Mf<T>::V V4;
+    typedef typename lanes::Vec16<T>::type V;
+    typedef typename lanes::Vec16u<T>::type Vu;
+    constexpr int B = CP_B, E = 16 / (int)sizeof(T), P = B + E;   // LDS pitch: 16-byte rows
+    __shared__ __align__(16) T Ls[5][B * P];   // the waves' row groups; [4]: the diagonal rows
+    __shared__ int s_last, s_fail;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l16 = lane & 15, grp = lane >> 4, l32 = lane & 31;
+    const bool low = lane < 32;
+    T *D = g.A + (long)g.k0 * g.lda + g.k0;
+    const int chunk0 = g.kb + B * (int)blockIdx.x;   // first of this workgroup's rows of A21, from k0
+    const int rows = g.n - g.k0;
+    // row group of a wave's upper lanes: its first row from k0, and the rows that exist
+    const int group0 = wave < 3 ? B * (wave + 1) : chunk0;
+    const int glimit = wave < 3 ? g.kb : rows;
+    // element (r, c) of the panel; outside the diagonal block the identity
+    T a[B];
+    {
+        const int r = low ? l32 : group0 + l32;
+        const bool ok = r < (low ? g.kb : glimit);
+        const T *src = D + (long)min(r, rows - 1) * g.lda;
+        if (g.kb >= B) {
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int i = min(i0 + q * (NT / 64), kb - 1);
+            for (int c = 0; c < B; c += E) {
+                const Vu v = *reinterpret_cast<const Vu *>(src + c);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) v[q][h] = D[(long)i * lda + min(lane + 64 * h, i)];
+                for (int e = 0; e < E; ++e) a[c + e] = ok ? v[e] : (T)0;
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < B; ++c) a[c] = (ok && c < g.kb) ? src[c] : (T)0;
         }
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int i = i0 + q * (NT / 64);
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-                if (i < kb && lane + 64 * h <= i) S[pk(i, lane + 64 * h)] = v[q][h];
+        for (int c = 0; c < B; ++c) {
+            if (low && c > l32) a[c] = (T)0;
+            if (low && !ok && c == l32) a[c] = (T)1;
         }
     }
+    // the later columns of the group, blocks 1 .. own, in the matrix-core layout
+    const int own = wave < 3 ? wave + 1 : 3;
+    V4 C[3][2][2];
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+        if (b < own)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int r = group0 + 16 * i + Mf<T>::row(grp, q), c = B * (b + 1) + 16 * j + l16;
+                        const bool ok = r < glimit && c < g.kb && (wave == 3 || c <= r);
+                        const T v = D[(long)min(r, rows - 1) * g.lda + min(c, g.kb - 1)];
+                        C[b][i][j][q] = ok ? v : (T)(wave < 3 && r == c ? 1 : 0);
+                    }
+    __builtin_amdgcn_s_waitcnt(0);
     if (t == 0) s_fail = 0;
     __syncthreads();
-    for (int jb = 0; jb < kb; jb += PB) {
-        const int pw = min(PB, kb - jb), je = jb + pw;
-        // A. the diagonal block
-        if (wave == 0) {
-            const int i = lane;
-            T a[PB];
+    if (t == 0) {
+        int last = 1;
+        if (gridDim.x > 1) {
+            last = __hip_atomic_fetch_add(g.arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                   (int)gridDim.x - 1;
+            if (last) __hip_atomic_store(g.arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        s_last = last;
+    }
 #pragma unroll
-            for (int c = 0; c < PB; ++c) a[c] = (i < pw && c <= i) ? S[pk(jb + i, jb + c)] : (T)0;
-            bool ok = true;
-            int fail_row = -1;
-            T fail_val = (T)0;
-#pragma unroll
-            for (int j = 0; j < PB; ++j) {
-                if (ok && j < pw) {
-                    const T dv = readlane_t<T>(a[j], j);
-                    if (!(dv > (T)0)) {
-                        ok = false;
-                        fail_row = jb + j;
-                        fail_val = dv;
-                    } else {
-                        const T d = sqrt(dv);
-                        a[j] = (i == j) ? d : (i > j ? a[j] / d : a[j]);
-                        T *cb = colb[j & 1];
-                        if (i < PB) cb[i] = a[j];
-                        wave_sync();
-                        // rows at or above j take a zero multiplier instead of a
-                        // select per column (a - 0 * l is a: l is finite)
-                        const T lj = i > j ? a[j] : (T)0;
-#pragma unroll
-                        for (int c = j + 1; c < PB; ++c) a[c] -= lj * cb[c];
-                    }
+    for (int jb = 0; jb < 4; ++jb) {
+        if (B * jb >= g.kb) break;
+        const bool active = wave == 3 || wave >= jb;   // the wave's group lies below the diagonal rows
+        if (active) {
+            T dv;
+            const int f = chol_columns<T, 0>(a, dv);
+            if (f >= 0) {
+                if (lane == 0) s_fail = 1;
+                if (wave == 3 && lane == 0 && blockIdx.x == 0) {
+                    *g.info = g.k0 + B * jb + f + 1;
+                    *g.info_val = (double)dv;
                 }
             }
+            if (!low || wave == 3) {
+                T *dst = Ls[low ? 4 : wave] + l32 * P;
 #pragma unroll
-            for (int c = 0; c < PB; ++c)
-                if (i < pw && c <= i) S[pk(jb + i, jb + c)] = a[c];
-            if (i < PB)
+                for (int c = 0; c < B; c += E) {
+                    V v;
 #pragma unroll
-                for (int c = 0; c < PB; ++c) Dsq[i][c] = a[c];
-            if (!ok && lane == 0) {
-                s_fail = 1;
-                *info = k0 + fail_row + 1;
-                *info_val = (double)fail_val;
+                    for (int e = 0; e < E; ++e) v[e] = a[c + e];
+                    *reinterpret_cast<V *>(dst + c) = v;
+                }
             }
         }
         __syncthreads();
         if (s_fail) return;
-        if (je >= kb) break;
-        // B. rows below: x L_jj^T = a, x_c = (a_c - sum_{q<c} x_q L[c][q]) / L[c][c]
-        //    (left-looking, four partial sums to shorten the chain).  Every
-        //    address is one base plus a constant: past pw the loads read the
-        //    padding after the triangle or stale entries, and the values they
-        //    give are masked before anything is stored.
-        // (kb <= 128, so at most 96 rows: one per thread — a loop over rows
-        // would let the compiler hoist the diagonal block's 528 loads out of it)
-        if (je + t < kb) {
-            const int r = je + t;
-            T *xr = S + pk(r, jb);
-            T x[PB];
+        // out: 256-byte (FP64) row segments; the diagonal block by the last arrival
+        auto write_out = [&](const T *src, int r0, int limit) {
+            constexpr int LPR = B / E, RPI = 64 / LPR;   // lanes per row, rows per store
 #pragma unroll
-            for (int c = 0; c < PB; ++c) {
-                const T v = xr[c];
-                x[c] = c < pw ? v : (T)0;
-            }
+            for (int i = 0; i < B / RPI; ++i) {
+                const int rr = RPI * i + lane / LPR, c = E * (lane % LPR), cc = B * jb + c;
+                const V v = *reinterpret_cast<const V *>(src + rr * P + c);
+                if (r0 + rr < limit) {
+                    T *dst = D + (long)(r0 + rr) * g.lda + cc;
+                    if (cc + E <= g.kb) *reinterpret_cast<Vu *>(dst) = v;
+                    else
 #pragma unroll
-            for (int c = 0; c < PB; ++c) {
-                // row c of the block, addressed through an offset the compiler
-                // sees only once x[c - 2] exists: its loads then overlap the
-                // previous column's division, and 528 loads are never in flight
-                // (or in registers) at once
-                int off = c * (PB + 1);
-                if (c >= 2) asm volatile("" : "+v"(off) : "v"(x[c - 2]));
-                const T *drow = &Dsq[0][0] + off;
-                T sp[4] = {x[c], (T)0, (T)0, (T)0};
-#pragma unroll
-                for (int q = 0; q < c; ++q) sp[q & 3] -= x[q] * drow[q];
-                const T v = ((sp[0] + sp[1]) + (sp[2] + sp[3])) / drow[c];
-                x[c] = c < pw ? v : (T)0;
-            }
-#pragma unroll
-            for (int c = 0; c < PB; ++c)
-                if (c < pw) xr[c] = x[c];
-        }
-        __syncthreads();
-        // C. S[r][c] -= sum_k S[r][jb+k] S[c][jb+k], je <= c <= r < kb, 16 x 16 tiles
-        {
-            const int lr = lane & 15, lk = lane >> 4;
-            const int nt = (kb - je + 15) / 16, ntiles = nt * (nt + 1) / 2;
-            for (int tile = wave; tile < ntiles; tile += NT / 64) {
-                int ti = 0;
-                while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
-                const int tj = tile - ti * (ti + 1) / 2;
-                const int r0 = je + 16 * ti, c0 = je + 16 * tj;
-                const int ra = min(r0 + lr, kb - 1), ca = min(c0 + lr, kb - 1);
-                typename MV<T>::V acc = {0, 0, 0, 0};
-                const T *ar = S + pk(ra, jb) + lk, *br = S + pk(ca, jb) + lk;
-                T av[PB / 4], bv[PB / 4];
-#pragma unroll
-                for (int k = 0; k < PB / 4; ++k) {
-                    const bool kk = 4 * k + lk < pw;
-                    const T x = ar[4 * k], y = br[4 * k];
-                    av[k] = kk ? x : (T)0;
-                    bv[k] = kk ? y : (T)0;
-                }
-#pragma unroll
-                for (int k = 0; k < PB / 4; ++k) acc = MV<T>::mfma(av[k], bv[k], acc);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int r = r0 + MV<T>::row(lk, q), c = c0 + lr;
-                    if (r < kb && c <= r) S[pk(r, c)] -= acc[q];
+                        for (int e = 0; e < E; ++e)
+                            if (cc + e < g.kb) dst[e] = v[e];
                 }
             }
+        };
+        if (wave == 3) write_out(Ls[3], chunk0, rows);
+        if (s_last) {
+            if (wave == 3) write_out(Ls[4], B * jb, g.kb);
+            else if (active) write_out(Ls[wave], group0, g.kb);
         }
-        __syncthreads();
-    }
-    for (int i = wave; i < kb; i += NT / 64)
-        for (int j = lane; j <= i; j += 64) D[(long)i * lda + j] = S[pk(i, j)];
-}
-
-// L21 = A21 L11^-T for rows [r0, r0 + nrows): each row x solves x L11^T = a,
-// i.e. x_j = (a_j - sum_{q<j} x_q L11[j][q]) / L11[j][j].
-template <typename T>
-__global__ __launch_bounds__(NT) void trsm_rltn_kernel(T *A, long lda, int k0, int kb, int r0, int nrows,
-                                                       const int *info)
-{
-    if (*info != 0) return;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    T *Ls = reinterpret_cast<T *>(smem_raw);        // packed lower incl. diagonal: row i at i*(i+1)/2
-    T *Bs = Ls + (size_t)kb * (kb + 1) / 2;         // kb x 65 (transposed strip: Bs[j*65 + row])
-    const int t = threadIdx.x, lane = t & 63, rg = t >> 6;
-    const T *L = A + (long)k0 * lda + k0;
-    for (int i = rg; i < kb; i += NT / 64) {
-        T *dst = Ls + (size_t)i * (i + 1) / 2;
-        for (int j = lane; j <= i; j += 64) dst[j] = L[(long)i * lda + j];
-    }
-    const int rbase = r0 + blockIdx.x * 64;
-    {
-        // the 64 x kb row strip, transposed into Bs[j*65 + r], 8 loads in flight per thread
-        const int vrows = min(64, r0 + nrows - rbase);
-        constexpr int U = 8;
-        for (int b = threadIdx.x; b < 64 * kb; b += U * NT) {
-            T v[U];
+        if (B * (jb + 1) >= g.kb) break;
+        // C -= L L^T on the later blocks; k-order: lane group grp, step i -> k = 8 grp + i
+        if (active) {
+            T lf[2][8];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int idx = b + u * NT, r = idx / kb, j = idx - r * kb;
-                v[u] = (idx < 64 * kb && r < vrows) ? A[(long)(rbase + r) * lda + k0 + j] : (T)0;
-            }
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int idx = b + u * NT, r = idx / kb, j = idx - r * kb;
-                if (idx < 64 * kb) Bs[j * 65 + r] = v[u];
-            }
-        }
-    }
-    __syncthreads();
-    for (int jb = 0; jb < kb; jb += 8) {
-        const int je = min(jb + 8, kb);
-        if (rg == 0) {
-            // the 8 columns of the block in registers: x_j = (b_j - sum_q L[j][q] x_q) / L[j][j]
-            T x[8];
+                for (int k = 0; k < 8; k += E) {
+                    const V v = *reinterpret_cast<const V *>(Ls[wave] + (16 * i + l16) * P + 8 * grp + k);
 #pragma unroll
-            for (int q = 0; q < 8; ++q) x[q] = (jb + q < je) ? Bs[(jb + q) * 65 + lane] : (T)0;
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                if (jb + q < je) {
-                    const T *Lj = Ls + (size_t)(jb + q) * (jb + q + 1) / 2 + jb;
-#pragma unroll
-                    for (int pp = 0; pp < q; ++pp) x[q] -= Lj[pp] * x[pp];
-                    x[q] = x[q] / Lj[q];
-                    Bs[(jb + q) * 65 + lane] = x[q];
+                    for (int e = 0; e < E; ++e) lf[i][k + e] = -v[e];
                 }
+#pragma unroll
+            for (int b = jb; b < 3; ++b)
+                if (b < own) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        T rf[8];
+#pragma unroll
+                        for (int k = 0; k < 8; k += E) {
+                            const V v = *reinterpret_cast<const V *>(Ls[b] + (16 * j + l16) * P + 8 * grp + k);
+#pragma unroll
+                            for (int e = 0; e < E; ++e) rf[k + e] = v[e];
+                        }
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+#pragma unroll
+                            for (int k = 0; k < 8; ++k) C[b][i][j] = Mf<T>::mac(lf[i][k], rf[k], C[b][i][j]);
+                    }
+                }
+        }
+        __syncthreads();
+        // the next step's columns back to rows, through LDS
+        if (active && jb < own) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        Ls[wave][(16 * i + Mf<T>::row(grp, q)) * P + 16 * j + l16] = C[jb < 3 ? jb : 0][i][j][q];
+        }
+        __syncthreads();
+        if (wave == 3 || wave >= jb + 1) {
+            const T *src = Ls[low ? jb : wave] + l32 * P;
+#pragma unroll
+            for (int c = 0; c < B; c += E) {
+                const V v = *reinterpret_cast<const V *>(src + c);
+#pragma unroll
+                for (int e = 0; e < E; ++e) a[c + e] = low && c + e > l32 ? (T)0 : v[e];
             }
         }
         __syncthreads();
-        T x[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) x[q] = (jb + q < je) ? Bs[(jb + q) * 65 + lane] : (T)0;
-        // later columns, four per wave at a time (all loads issued before the arithmetic)
-        for (int j0 = je + rg; j0 < kb; j0 += 4 * (NT / 64)) {
-            T acc[4], lv[4][8];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = min(j0 + u * (NT / 64), kb - 1);
-                acc[u] = Bs[j * 65 + lane];
-                const T *Lj = Ls + (size_t)j * (j + 1) / 2 + jb;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) lv[u][q] = (jb + q < je) ? Lj[q] : (T)0;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int q = 0; q < 8; ++q) acc[u] -= lv[u][q] * x[q];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (j0 + u * (NT / 64) < kb) Bs[(j0 + u * (NT / 64)) * 65 + lane] = acc[u];
-        }
-        __syncthreads();
-    }
-    for (int r = rg; r < 64; r += NT / 64) {
-        const int gr = rbase + r;
-        if (gr < r0 + nrows)
-            for (int j = lane; j < kb; j += 64) A[(long)gr * lda + k0 + j] = Bs[j * 65 + r];
-    }
-}
-
-// Linv = L11^-1 of the 128 x 128 FP64 diagonal block (lower, non-unit), for
-// the TRSM as a product L21 = A21 Linv^T.  Blocks of 32:
-//   1. wave w inverts diagonal block w, lane c computing column c by forward
-//      substitution in registers (true division by the diagonal);
-//   2. block rows i = 1..3 in order, for each j < i:
-//      T = sum_{k=j}^{i-1} L_ik Linv_kj, then Linv_ij = -Linv_ii T
-//      (all 256 threads, one row x 4 columns of the 32 x 32 block each);
-//   3. Linv (lower, zeros above) to global, row stride 128.
-// The inverse's ten lower blocks and one T block live in LDS (88 KiB, so the
-// kernel fits on a CU beside one workgroup of the trailing update running on
-// the other stream); L is read from global memory (cached).
-constexpr int TI64 = 128, TB64 = 32;
-__device__ __forceinline__ int blk64(int i, int j) { return (i * (i + 1) / 2 + j) * TB64 * TB64; }
-__global__ __launch_bounds__(NT) void trtri_lower64_kernel(const double *L, long ldl, double *Linv, const int *info)
-{
-    if (*info != 0) return;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    double *X = reinterpret_cast<double *>(smem_raw);   // 10 blocks of 32 x 32
-    double *Ts = X + 10 * TB64 * TB64;                   // 32 x 32
-    const int t = threadIdx.x, lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    {
-        const double *D = L + (long)(TB64 * wave) * ldl + TB64 * wave;
-        const int c = lane;
-        double x[TB64];
-#pragma unroll
-        for (int i = 0; i < TB64; ++i) {
-            double sacc = (i == c) ? 1.0 : 0.0;
-#pragma unroll
-            for (int j = 0; j < i; ++j) sacc -= D[(long)i * ldl + j] * x[j];
-            x[i] = sacc / D[(long)i * ldl + i];
-        }
-        if (c < TB64)
-#pragma unroll
-            for (int i = 0; i < TB64; ++i) X[blk64(wave, wave) + i * TB64 + c] = x[i];
-    }
-    __syncthreads();
-    const int r = t >> 3, c4 = t & 7;   // this thread's row and four columns of a block
-    for (int i = 1; i < TI64 / TB64; ++i) {
-        const double *Lr = L + (long)(TB64 * i + r) * ldl;
-        for (int j = 0; j < i; ++j) {
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-            for (int k = j; k < i; ++k) {
-                const double *xk = X + blk64(k, j) + 4 * c4;
-                // the row's 32 entries of L_ik in one round trip to memory
-                double lv[TB64];
-#pragma unroll
-                for (int q = 0; q < TB64; ++q) lv[q] = Lr[TB64 * k + q];
-#pragma unroll
-                for (int q = 0; q < TB64; ++q)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[e] = fma(lv[q], xk[q * TB64 + e], acc[e]);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) Ts[r * TB64 + 4 * c4 + e] = acc[e];
-            __syncthreads();
-            const double *dr = X + blk64(i, i) + r * TB64;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = 0.0;
-            for (int q = 0; q <= r; ++q) {
-                const double a = dr[q];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] = fma(a, Ts[q * TB64 + 4 * c4 + e], acc[e]);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) X[blk64(i, j) + r * TB64 + 4 * c4 + e] = -acc[e];
-            __syncthreads();
-        }
-    }
-    for (int e = t; e < TI64 * TI64; e += NT) {
-        const int rr = e / TI64, cc = e % TI64;
-        Linv[e] = cc <= rr ? X[blk64(rr / TB64, cc / TB64) + (rr % TB64) * TB64 + cc % TB64] : 0.0;
     }
 }
 
@@ -416,36 +340,14 @@ int scirs_potrf_device(int n, T *A, long lda, int kb, ScirsWork &w, hipStream_t 
     }
     for (int k0 = 0, p = 0; k0 < n; k0 += kb, ++p) {
         const int kbw = std::min(kb, n - k0);
-        // the packed triangle and PB elements of padding that reads past a
-        // partial column block may touch
-        const size_t lds_p = ((size_t)kbw * (kbw + 1) / 2 + 32) * sizeof(T);
-        if (int rc = scirs_allow_lds((const void *)potf2_kernel<T>, lds_p)) return rc;
-        hipLaunchKernelGGL(potf2_kernel<T>, dim3(1), dim3(NT), lds_p, stream,
-                           A, lda, k0, kbw, w.info, w.info_val);
         const int rest = n - k0 - kbw;
+        CholPanelArgs<T> pa;
+        pa.A = A; pa.lda = lda; pa.k0 = k0; pa.kb = kbw; pa.n = n;
+        pa.arrive = w.sub_arrive; pa.info = w.info; pa.info_val = w.info_val;
+        hipLaunchKernelGGL(chol_panel_kernel<T>, dim3(std::max(1, (rest + CP_B - 1) / CP_B)), dim3(NT), 0,
+                           stream, pa);
+        SCIRS_HIP_CHECK(hipGetLastError());
         if (rest > 0) {
-            static const bool inv_trsm = [] {
-                const char *v = getenv("SCIRS_GPU_CHOL_INV_TRSM");
-                return !(v && *v && atoi(v) == 0);
-            }();
-            if (std::is_same<T, double>::value && kbw == TI64 && w.linv64 && inv_trsm) {
-                // L21 = A21 L11^-T as a product on the matrix cores: L11^-1 by one
-                // workgroup, then one 128-row tile of A21 per workgroup, in place
-                const size_t lds_i = (size_t)11 * TB64 * TB64 * sizeof(double);
-                if (int rc = scirs_allow_lds((const void *)trtri_lower64_kernel, lds_i)) return rc;
-                hipLaunchKernelGGL(trtri_lower64_kernel, dim3(1), dim3(NT), lds_i, stream,
-                                   (const double *)(A + (long)k0 * lda + k0), lda, w.linv64, (const int *)w.info);
-                SCIRS_HIP_CHECK(hipGetLastError());
-                double *A21 = (double *)(A + (long)(k0 + kbw) * lda + k0);
-                if (int rc = scirs_launch_dgemm_assign_t(rest, TI64, TI64, A21, lda, w.linv64, TI64, A21, lda,
-                                                         (const int *)w.info, stream))
-                    return rc;
-            } else {
-                const size_t lds = ((size_t)kbw * (kbw + 1) / 2 + (size_t)kbw * 65) * sizeof(T);
-                if (int rc = scirs_allow_lds((const void *)trsm_rltn_kernel<T>, lds)) return rc;
-                hipLaunchKernelGGL(trsm_rltn_kernel<T>, dim3((rest + 63) / 64), dim3(NT), lds, stream,
-                                   A, lda, k0, kbw, k0 + kbw, rest, (const int *)w.info);
-            }
             const T *L21 = A + (long)(k0 + kbw) * lda + k0;
             T *A22 = A + (long)(k0 + kbw) * lda + k0 + kbw;
             const int nn = lookahead ? std::min(kb, rest) : rest;   // columns updated on the main stream
