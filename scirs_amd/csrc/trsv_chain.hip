@@ -127,13 +127,39 @@ __device__ bool poll_vals(const u64 *src, int nvalid, unsigned seq, T (&v)[NV], 
     }
 }
 
+// This workgroup's place in the launch's order.  Every workgroup takes one, also
+// when there is nothing to solve (info set: -1), and the last to do so clears the
+// counter: it is zero between launches, and no launch of its own (4.6 us) clears it.
+__device__ __forceinline__ int take_ticket(int *ticket, const int *info)
+{
+    const int b = atomicAdd(ticket, 1);
+    if (b == (int)gridDim.x - 1) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return info && *info != 0 ? -1 : b;
+}
+
+// 64 rows of 64 elements into LDS (pitch LDP), 32 loads in flight per lane; zero past
+// rows x cols
+template <typename T>
+__device__ __forceinline__ void stage_tile(T *dst, const T *src, long ld, int rows, int cols)
+{
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i0 = 0; i0 < TB; i0 += 32) {
+        T v[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u)
+            v[u] = (i0 + u < rows && lane < cols) ? src[(long)(i0 + u) * ld + lane] : (T)0;
+#pragma unroll
+        for (int u = 0; u < 32; ++u) dst[(i0 + u) * LDP + lane] = v[u];
+    }
+}
+
 template <typename T, int QB, bool LOWER, bool UNIT>
 __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A, long lda, T *X, long ldx, int n,
                                                          int nrhs, u64 *xch, unsigned seq, int *ticket, int *abort,
                                                          unsigned spin_limit, int *info,
                                                          const T *__restrict__ dinv, const T *__restrict__ dmt)
 {
-    if (info && *info != 0) return;
     // blockIdx.y: a group of QB right-hand sides, an independent chain with its
     // own ticket and exchange region (the groups run side by side)
     const int grp = blockIdx.y;
@@ -148,8 +174,9 @@ __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A
     T *part = Lt + TB * LDP;                    // [3][TB][QB] partial sums of waves 1-3
     __shared__ int s_ticket;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (t == 0) s_ticket = atomicAdd(ticket, 1);
+    if (t == 0) s_ticket = take_ticket(ticket, info);
     __syncthreads();
+    if (s_ticket < 0) return;
     const int b = s_ticket;                      // position in dependency order
     const int nblk = (n + TB - 1) / TB;
     const int p = LOWER ? b : nblk - 1 - b;      // block row solved here
@@ -204,23 +231,13 @@ __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A
     } else {
         // ---- wave 0: stage the diagonal block (or its inverse) and the last
         //      dependency's tile (coalesced rows)
-        if (dinv) {
-            const T *Dp = dinv + (size_t)p * TB * TB;
-            for (int i = 0; i < TB; ++i) Ld[i * LDP + lane] = Dp[i * TB + lane];
-        } else {
-            for (int i = 0; i < TB; ++i)
-                Ld[i * LDP + lane] = (i < bs && lane < bs) ? A[(long)(r0 + i) * lda + r0 + lane] : (T)0;
-        }
+        if (dinv) stage_tile(Ld, dinv + (size_t)p * TB * TB, (long)TB, TB, TB);
+        else stage_tile(Ld, A + (long)r0 * lda + r0, lda, bs, bs);
         if (b > 0) {
             const int cb = LOWER ? b - 1 : nblk - b;
             const int c0 = cb * TB, cs = min(TB, n - c0);
-            if (dmt) {
-                const T *Mp = dmt + (size_t)p * TB * TB;   // D^-1 times the last tile
-                for (int i = 0; i < TB; ++i) Lt[i * LDP + lane] = Mp[i * TB + lane];
-            } else {
-                for (int i = 0; i < TB; ++i)
-                    Lt[i * LDP + lane] = (i < bs && lane < cs) ? A[(long)(r0 + i) * lda + c0 + lane] : (T)0;
-            }
+            if (dmt) stage_tile(Lt, dmt + (size_t)p * TB * TB, (long)TB, TB, TB);   // D^-1 times the last tile
+            else stage_tile(Lt, A + (long)r0 * lda + c0, lda, bs, cs);
         }
     }
     __syncthreads();
@@ -262,6 +279,37 @@ __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A
 #pragma unroll
         for (int q = 0; q < QB; ++q) s[q] = xo[q];
     } else {
+    // The diagonal and its reciprocal, one row per lane, before the last
+    // dependency arrives: the division then costs three dependent operations
+    // per row instead of about thirty (FP64, n = 1000, one right-hand side:
+    // 155 us for the 16 links with a division per row, 99 us so).  FP64: the
+    // correctly rounded quotient (reciprocal to an ulp, one residual
+    // correction), as the reference divides; where the block has a diagonal
+    // whose reciprocal nears the subnormals, true division.  FP32 multiplies
+    // by the reciprocal.
+    constexpr bool EXACT = sizeof(T) == 8;
+    T dl = (T)1, rl = (T)1;
+    bool divide = false;
+    if (!UNIT) {
+        if (lane < bs) dl = Ld[lane * LDP + lane];
+        if constexpr (EXACT) {
+            rl = __builtin_amdgcn_rcp(dl);
+            rl = fma(rl, fma(-dl, rl, 1.0), rl);
+            rl = fma(rl, fma(-dl, rl, 1.0), rl);
+            divide = __any(!(fabs(dl) > 0x1p-960 && fabs(dl) < 0x1p+960));
+        } else {
+            rl = (T)1 / dl;
+        }
+    }
+    auto quotient = [&](T v) -> T {
+        if constexpr (UNIT) return v;
+        if constexpr (!EXACT) return v * rl;
+        else {
+            if (__builtin_expect(divide, 0)) return v / dl;
+            const T x = v * rl, y = fma(fma(-x, dl, v), rl, x);
+            return fabs(x) < __builtin_huge_val() ? y : x;   // infinite or NaN: as it came
+        }
+    };
     if (b > 0) {
         const int cb = LOWER ? b - 1 : nblk - b;
         const int c0 = cb * TB;
@@ -270,12 +318,21 @@ __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A
                                  abort, info))
             failed = true;
         if (failed) return;
+        // two partial sums: half the dependent chain
+        T s2[QB];
 #pragma unroll
-        for (int k = 0; k < TB; ++k) {
-            const T l = Lt[lane * LDP + k];
+        for (int q = 0; q < QB; ++q) s2[q] = (T)0;
 #pragma unroll
-            for (int q = 0; q < QB; ++q) s[q] -= l * readlane(xk[q], k);
+        for (int k = 0; k < TB; k += 2) {
+            const T l0 = Lt[lane * LDP + k], l1 = Lt[lane * LDP + k + 1];
+#pragma unroll
+            for (int q = 0; q < QB; ++q) {
+                s[q] -= l0 * readlane(xk[q], k);
+                s2[q] -= l1 * readlane(xk[q], k + 1);
+            }
         }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) s[q] += s2[q];
     }
     if (failed) return;
     if (dinv) {
@@ -293,44 +350,25 @@ __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A
 #pragma unroll
         for (int q = 0; q < QB; ++q) s[q] = xo[q];
     } else {
-    // FP64 divides by the diagonal as the reference does; FP32 multiplies by a
-    // reciprocal each lane computes up front, which keeps the division off the
-    // 64-step dependent chain (the FP32 factors only precondition refinement).
-    constexpr bool EXACT = sizeof(T) == 8;
-    const T rinv = (!UNIT && !EXACT && lane < bs) ? (T)1 / Ld[lane * LDP + lane] : (T)1;
-    if (LOWER) {
+        // 64 steps: row k's value to every lane, which keeps it as its own x (lane k) and
+        // subtracts its multiple (rows already solved change too, but are not read again;
+        // rows past bs hold zeros)
+        T xo[QB];
 #pragma unroll
-        for (int k = 0; k < TB; ++k) {
-            if (k < bs) {
-                const T l = Ld[lane * LDP + k];
-                const T d = Ld[k * LDP + k];
-                const T rk = readlane(rinv, k);
+        for (int q = 0; q < QB; ++q) xo[q] = (T)0;
 #pragma unroll
-                for (int q = 0; q < QB; ++q) {
-                    T x = readlane(s[q], k);
-                    if (!UNIT) x = EXACT ? x / d : x * rk;
-                    if (lane == k) s[q] = x;
-                    else if (lane > k) s[q] -= l * x;
-                }
+        for (int kk = 0; kk < TB; ++kk) {
+            const int k = LOWER ? kk : TB - 1 - kk;
+            const T l = Ld[lane * LDP + k];
+#pragma unroll
+            for (int q = 0; q < QB; ++q) {
+                const T x = readlane(quotient(s[q]), k);
+                xo[q] = lane == k ? x : xo[q];
+                s[q] -= l * x;
             }
         }
-    } else {
 #pragma unroll
-        for (int k = TB - 1; k >= 0; --k) {
-            if (k < bs) {
-                const T l = Ld[lane * LDP + k];
-                const T d = Ld[k * LDP + k];
-                const T rk = readlane(rinv, k);
-#pragma unroll
-                for (int q = 0; q < QB; ++q) {
-                    T x = readlane(s[q], k);
-                    if (!UNIT) x = EXACT ? x / d : x * rk;
-                    if (lane == k) s[q] = x;
-                    else if (lane < k) s[q] -= l * x;
-                }
-            }
-        }
-    }
+        for (int q = 0; q < QB; ++q) s[q] = xo[q];
     }
     }
     if (lane < bs) {
@@ -364,7 +402,6 @@ __global__ __launch_bounds__(NTP) void trsv_pair_kernel(const float *__restrict_
                                                         unsigned spin_limit, int *info,
                                                         const float *__restrict__ dinv, const float *__restrict__ dm)
 {
-    if (info && *info != 0) return;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     float *Mx = reinterpret_cast<float *>(smem_raw);   // [PLM][TB][LDP]
     float *part = Mx + PLM * TB * LDP;                 // [6][TB] partial sums of waves 2-7
@@ -373,9 +410,10 @@ __global__ __launch_bounds__(NTP) void trsv_pair_kernel(const float *__restrict_
     u64 *xe_w = reinterpret_cast<u64 *>(part + 6 * TB);
     __shared__ int s_ticket;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (t == 0) s_ticket = atomicAdd(ticket, 1);
+    if (t == 0) s_ticket = take_ticket(ticket, info);
     if (t < TB) xe_w[t] = 0ull;
     __syncthreads();
+    if (s_ticket < 0) return;
     const int q = s_ticket;
     const int nblk = (n + TB - 1) / TB;
     const int e = 2 * q, o = e + 1;
@@ -534,8 +572,7 @@ int launch_chain(int n, int nr, const T *A, long lda, T *X, long ldx, ScirsWork 
         int rc = scirs_allow_lds((const void *)kern, lds);
         if (rc) return rc;
     }
-    int rc = scirs_fill_int(w.ticket, groups, 0, s);
-    if (rc) return rc;
+    int rc = SCIRS_OK;
     unsigned seq = 0;
     if ((rc = scirs_next_seq(w, 512u, s, &seq))) return rc;
     const int nblk = (n + TB - 1) / TB;
@@ -562,7 +599,6 @@ int launch_pair(int n, const float *A, long lda, float *X, ScirsWork &w, hipStre
     const size_t lds = ((size_t)PLM * TB * LDP + 8 * (size_t)TB) * sizeof(float);
     int rc = scirs_allow_lds((const void *)kern, lds);
     if (rc) return rc;
-    if ((rc = scirs_fill_int(w.ticket, 1, 0, s))) return rc;
     unsigned seq = 0;
     if ((rc = scirs_next_seq(w, 512u, s, &seq))) return rc;
     const int nblk = (n + TB - 1) / TB;
