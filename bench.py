@@ -228,7 +228,7 @@ def make_batch(count, seed, torch):
 
 
 def bench_batched(args):
-    """20,000 uneven systems in one persistent launch vs. a per-matrix launch loop."""
+    """20,000 uneven systems in one call vs. a per-matrix launch loop."""
     import numpy as np
     import torch
     from scirs_amd import linalg as L
@@ -289,7 +289,7 @@ def bench_batched(args):
                             "note": "gesv_dev / posv_dev per system, timed on the first "
                                     f"{sample} systems and scaled to {args.batch}"},
         "speedup_vs_loop": t_loop / t,
-        "roofline": {"bound": "hbm", "kernel": "batched_solve_kernel", "achieved": roof_bw,
+        "roofline": {"bound": "hbm", "kernel": "batched_wave_kernel", "achieved": roof_bw,
                      "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": roof_bw / PEAK_HBM_GBS, "traffic": None,
                      "algorithmic_bytes": bytes_alg},
     }

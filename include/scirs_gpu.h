@@ -253,7 +253,7 @@ typedef struct scirs_batch_info {
     double max_backward_error;   /* over the systems with status 0                   */
     double time_ms;              /* device time of the batched launch                */
     double total_ms;             /* wall time of the call                            */
-    int32_t wave_max;            /* systems with n <= wave_max ran one per wave      */
+    int32_t wave_max;            /* FP64 systems with n <= wave_max ran one per wave */
     int32_t graph_replayed;      /* 1 when the launch replayed a cached hipGraph     */
 } scirs_batch_info;
 int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *nrhs, const unsigned char *spd,

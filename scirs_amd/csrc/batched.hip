@@ -13,17 +13,18 @@
 // r = b - A x from the FP64 input, correction with the FP32 factors — until
 // the normwise backward error of every right-hand side is <= tol.  A system
 // whose FP32 factorisation breaks down, or whose refinement stalls, is
-// factored again in FP64 by the same code (the breakdown is then decided in
-// FP64, as the reference decides it).
+// factored again in FP64 (the breakdown is then decided in FP64, as the
+// reference decides it).
 //
-// Scheduling: the host sorts the systems by decreasing n into a queue;
-// workgroups pop queue entries with an atomic counter.  Entries with n >
-// wave_max are processed by the whole 256-thread workgroup; smaller ones are
-// processed one per wave (four per workgroup pop).  The crossover is a
-// runtime argument picked by the batched autotuner (api side).
+// Scheduling: the host sorts the systems by decreasing n.  One launch takes
+// every system through FP32 and the refinement, one wave each
+// (batched_wave.hpp); it marks those that need FP64, and a second launch takes
+// these from a queue: n > wave_max by a 256-thread workgroup, smaller ones one
+// per wave.  Without any it ends at once.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "prof.hpp"
+#include "batched_wave.hpp"
 
 namespace {
 
@@ -34,7 +35,7 @@ constexpr int NMAX = 256;       // largest system handled
 struct BatchDesc {
     int n, nrhs, spd, pad;
     long offA, offB;            // element offsets of A (n x n) and B/X (n x nrhs) in the packed buffers
-    long offW;                  // element offset (FP64 units) of the factor workspace (n x n)
+    long offW;                  // element offset (FP64 units) of the factor workspace
 };
 
 struct BatchArgs {
@@ -42,14 +43,14 @@ struct BatchArgs {
     const int *order;           // queue: system indices sorted by decreasing n
     int batch;
     const double *A; const double *B; double *X;
-    double *work;               // factor workspace, n*n doubles per system
+    double *work;               // factor workspace, work_doubles(n) per system
     int *perm;                  // n ints per system (offset = offA / n ... use offB-like index: offP)
     const long *offP;
     int *status;                // per system: 0 ok, k>0 breakdown column/row, -5 not converged
     int *iters;                 // per system: refinement steps
     double *bwd;                // per system: final backward error
-    unsigned *counter;          // queue head, reset to 0 before each launch
-    int wave_max;               // n <= wave_max -> one wave per system
+    unsigned *counter;          // [0] queue head, [1] a system needs FP64; cleared ahead of the launches
+    int wave_max;               // FP64: n <= wave_max -> one wave per system
     int max_iter;
     double tol_scale;           // tol = tol_scale * n * 2^-53 (per system)
 };
@@ -105,7 +106,7 @@ __device__ __forceinline__ T team_max(T v, T *red_v)
 // LDS (pan: n x (NB+1)), the trailing update reads the panel from LDS.
 // Returns 0 or the 1-based breakdown column.
 template <int TEAM, typename T>
-__device__ int team_getrf(int n, T *M, int *perm, T *pan, T *red_v, int *red_i, int tid, T *ustage)
+__device__ int team_getrf(int n, T *M, int *perm, T *pan, T *red_v, int *red_i, int tid)
 {
     for (int i = tid; i < n; i += TEAM) perm[i] = i;
     const T eps = num_limits<T>::eps();
@@ -166,57 +167,22 @@ __device__ int team_getrf(int n, T *M, int *perm, T *pan, T *red_v, int *red_i, 
         const int c1 = k0 + kb;
         if (c1 >= n) continue;
         const int rows = n - c1, cols = n - c1;
-        if constexpr (sizeof(T) == 4) {
-        // U12 = L11^-1 A12 (rows k0..k0+kb): one column per thread, its kb
-            // entries loaded together into registers, the same subtraction order
-            // as the loop over i and q
-            for (int c = c1 + tid; c < n; c += TEAM) {
-                T u[NB];
-#pragma unroll
-                for (int i = 0; i < NB; ++i) u[i] = i < kb ? M[(long)(k0 + i) * n + c] : (T)0;
-#pragma unroll
-                for (int i = 1; i < NB; ++i) {
-                    // row i of L11 through an offset the compiler sees only once
-                    // u[i - 1] exists, so its loads are not all hoisted (they spill)
-                    int off = i * (NB + 1);
-                    asm volatile("" : "+v"(off) : "v"(u[i - 1]));
-                    const T *li = pan + off;
-                    T sv = u[i];
-#pragma unroll
-                    for (int q = 0; q < i; ++q) sv -= li[q] * u[q];
-                    u[i] = sv;
-                }
-#pragma unroll
-                for (int i = 0; i < NB; ++i) {
-                    if (i < kb) M[(long)(k0 + i) * n + c] = u[i];
-                    // rows past kb are zero in the staged copy (the panel's columns past kb are zero too)
-                    if (ustage) ustage[i * cols + (c - c1)] = i < kb ? u[i] : (T)0;
-                }
+        // U12 = L11^-1 A12 in memory (registers for 32 doubles would spill in this kernel)
+        for (int c = c1 + tid; c < n; c += TEAM)
+            for (int i = 1; i < kb; ++i) {
+                T sv = M[(long)(k0 + i) * n + c];
+                for (int q = 0; q < i; ++q) sv -= pan[i * (NB + 1) + q] * M[(long)(k0 + q) * n + c];
+                M[(long)(k0 + i) * n + c] = sv;
             }
-        } else {
-            // the FP64 fallback: the column in memory (registers for 32 doubles
-            // would spill in this kernel)
-            for (int c = c1 + tid; c < n; c += TEAM)
-                for (int i = 1; i < kb; ++i) {
-                    T sv = M[(long)(k0 + i) * n + c];
-                    for (int q = 0; q < i; ++q) sv -= pan[i * (NB + 1) + q] * M[(long)(k0 + q) * n + c];
-                    M[(long)(k0 + i) * n + c] = sv;
-                }
-        }
         team_sync<TEAM>();
-        // A22 -= L21 U12 (U12 from the staged copy when there is one)
+        // A22 -= L21 U12
         for (int w = tid; w < rows * cols; w += TEAM) {
             const int r = w / cols, c = w % cols;
             const T *lr = pan + (kb + r) * (NB + 1);
             T sv = (T)0;
-            if (ustage) {
 #pragma unroll 8
-                for (int q = 0; q < NB; ++q) sv += lr[q] * ustage[q * cols + c];
-            } else {
-#pragma unroll 8
-                for (int q = 0; q < NB; ++q)
-                    if (q < kb) sv += lr[q] * M[(long)(k0 + q) * n + c1 + c];
-            }
+            for (int q = 0; q < NB; ++q)
+                if (q < kb) sv += lr[q] * M[(long)(k0 + q) * n + c1 + c];
             M[(long)(c1 + r) * n + c1 + c] -= sv;
         }
     }
@@ -278,96 +244,8 @@ __device__ int team_potrf(int n, T *M, T *pan, int tid)
     return 0;
 }
 
-__device__ __forceinline__ double bcast_lane(double v, int q)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), q);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), q);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-// d <- op^-1 d with the factors in M (row-major, ld n); d in LDS (length n).
-// LU: L unit lower then U; Cholesky: L then L^T.  Blocks of NB rows: the
-// first wave solves the diagonal block (lane i = row i, the solved value
-// broadcast by readlane), then every thread takes one row outside the block
-// and removes the block's contribution.  Each row receives the same
-// subtractions, in the same order, as a column-by-column sweep.
-template <int TEAM, typename T, typename V>
-__device__ void team_subst(int n, const T *M, V *d, bool chol, int tid)
-{
-    const int lane = tid & 63;
-    const bool w0 = tid < 64;
-    // forward: L (unit for LU)
-    for (int k0 = 0; k0 < n; k0 += NB) {
-        const int kb = min(NB, n - k0);
-        if (w0) {
-            const int i = lane;
-            const bool in = i < kb;
-            const int ri = k0 + min(i, kb - 1);
-            V di = in ? d[k0 + i] : (V)0;
-            T lrow[NB];
-#pragma unroll
-            for (int q = 0; q < NB; ++q) lrow[q] = M[(long)ri * n + k0 + min(q, kb - 1)];
-            const V dg = (V)M[(long)ri * n + ri];
-#pragma unroll
-            for (int q = 0; q < NB; ++q) {
-                if (q < kb) {
-                    if (chol && i == q) di /= dg;
-                    const V xq = bcast_lane(di, q);
-                    if (in && i > q) di -= (V)lrow[q] * xq;
-                }
-            }
-            if (in) d[k0 + i] = di;
-        }
-        team_sync<TEAM>();
-        for (int r = k0 + kb + tid; r < n; r += TEAM) {
-            V sv = d[r];
-#pragma unroll 8
-            for (int q = 0; q < NB; ++q)
-                if (q < kb) sv -= (V)M[(long)r * n + k0 + q] * d[k0 + q];
-            d[r] = sv;
-        }
-        team_sync<TEAM>();
-    }
-    // backward: U (LU) or L^T (Cholesky), blocks from the bottom
-    for (int k0 = (n - 1) / NB * NB; k0 >= 0; k0 -= NB) {
-        const int kb = min(NB, n - k0);
-        if (w0) {
-            const int i = lane;
-            const bool in = i < kb;
-            const int ri = k0 + min(i, kb - 1);
-            V di = in ? d[k0 + i] : (V)0;
-            T urow[NB];
-#pragma unroll
-            for (int q = 0; q < NB; ++q) {
-                const int cq = k0 + min(q, kb - 1);
-                urow[q] = chol ? M[(long)cq * n + ri] : M[(long)ri * n + cq];
-            }
-            const V dg = (V)M[(long)ri * n + ri];
-#pragma unroll
-            for (int q = NB - 1; q >= 0; --q) {
-                if (q < kb) {
-                    if (i == q) di /= dg;
-                    const V xq = bcast_lane(di, q);
-                    if (in && i < q) di -= (V)urow[q] * xq;
-                }
-            }
-            if (in) d[k0 + i] = di;
-        }
-        team_sync<TEAM>();
-        for (int r = tid; r < k0; r += TEAM) {
-            V sv = d[r];
-#pragma unroll 8
-            for (int q = NB - 1; q >= 0; --q)
-                if (q < kb) sv -= (V)(chol ? M[(long)(k0 + q) * n + r] : M[(long)r * n + k0 + q]) * d[k0 + q];
-            d[r] = sv;
-        }
-        team_sync<TEAM>();
-    }
-}
-
-// The FP64 fallback's solve, column by column (d in LDS, length n): every thread reads the finished d[i], then the team
-// removes its contribution from the remaining entries (one sync per row).
+// d <- op^-1 d with the factors in M, column by column (d in LDS, length n): every thread reads the finished d[i], then
+// the team removes its contribution from the remaining entries (one sync per row).
 // LU: L unit lower then U; Cholesky: L then L^T.
 template <int TEAM, typename T, typename V>
 __device__ void team_subst_cols(int n, const T *M, V *d, bool chol, int tid)
@@ -390,10 +268,9 @@ __device__ void team_subst_cols(int n, const T *M, V *d, bool chol, int tid)
     }
 }
 
-// Solve one system with a team: FP32 factor + FP64 refinement, FP64 fallback.
+// Solve one system with a team, in FP64: factor + refinement.
 template <int TEAM>
-__device__ void team_solve(const BatchArgs &a, int sys, float *pan32, double *pan64, double *vec, double *red,
-                           float *redf, int *redi, int tid)
+__device__ void team_solve(const BatchArgs &a, int sys, double *pan, double *vec, double *red, int *redi, int tid)
 {
     const BatchDesc d = a.desc[sys];
     const int n = d.n, nrhs = d.nrhs;
@@ -401,8 +278,7 @@ __device__ void team_solve(const BatchArgs &a, int sys, float *pan32, double *pa
     const double *B = a.B + d.offB;
     double *X = a.X + d.offB;
     int *perm = a.perm + a.offP[sys];
-    double *W64 = a.work + d.offW;
-    float *W32 = reinterpret_cast<float *>(W64);
+    double *W = a.work + d.offW;
     const double tol = a.tol_scale * n * 0x1p-53;
 
     // ||A||_inf
@@ -414,34 +290,16 @@ __device__ void team_solve(const BatchArgs &a, int sys, float *pan32, double *pa
     }
     an = team_max<TEAM>(an, red);
 
-    int status = 0, it_used = 0;
+    int it_used = 0;
     double worst = 0.0;
-    for (int pass = 0; pass < 2; ++pass) {
-        const bool f64 = (pass == 1);
-        bool chol = d.spd != 0;
-        // copy A into the workspace and factor
-        int rc;
-        if (!f64) {
-            for (int idx = tid; idx < n * n; idx += TEAM) W32[idx] = (float)A[idx];
-            team_sync<TEAM>();
-            // U12 is staged in the half of the panel buffer an FP32 panel leaves free
-            rc = chol ? team_potrf<TEAM, float>(n, W32, pan32, tid)
-                      : team_getrf<TEAM, float>(n, W32, perm, pan32, redf, redi, tid,
-                                                pan32 + (size_t)(TEAM == NT ? NMAX : NMAX / 4) * (NB + 1));
-            if (rc != 0) continue;   // FP32 breakdown: the same factorisation decides in FP64
-        } else {
-            for (int idx = tid; idx < n * n; idx += TEAM) W64[idx] = A[idx];
-            team_sync<TEAM>();
-            if (chol) {
-                rc = team_potrf<TEAM, double>(n, W64, pan64, tid);
-            } else {
-                rc = team_getrf<TEAM, double>(n, W64, perm, pan64, red, redi, tid, nullptr);
-            }
-            if (rc != 0) { status = rc; break; }
-        }
+    const bool chol = d.spd != 0;
+    // copy A into the workspace and factor
+    for (int idx = tid; idx < n * n; idx += TEAM) W[idx] = A[idx];
+    team_sync<TEAM>();
+    const int status = chol ? team_potrf<TEAM, double>(n, W, pan, tid)
+                            : team_getrf<TEAM, double>(n, W, perm, pan, red, redi, tid);
+    if (status == 0) {
         // refinement for each right-hand side
-        worst = 0.0;
-        bool all_ok = true;
         for (int j = 0; j < nrhs; ++j) {
             for (int r = tid; r < n; r += TEAM) X[(long)r * nrhs + j] = 0.0;
             team_sync<TEAM>();
@@ -483,18 +341,12 @@ __device__ void team_solve(const BatchArgs &a, int sys, float *pan32, double *pa
                     for (int r = tid; r < n; r += TEAM) vec[r] = tmp[r];
                 }
                 team_sync<TEAM>();
-                if (f64) team_subst_cols<TEAM, double, double>(n, W64, vec, chol, tid);
-                else team_subst<TEAM, float, double>(n, W32, vec, chol, tid);
+                team_subst_cols<TEAM, double, double>(n, W, vec, chol, tid);
                 for (int r = tid; r < n; r += TEAM) X[(long)r * nrhs + j] += vec[r];
                 team_sync<TEAM>();
             }
             it_used = max(it_used, it);
             worst = fmax(worst, eta);
-            if (!(eta <= tol)) all_ok = false;
-        }
-        if (all_ok || f64) {
-            status = all_ok ? 0 : (f64 ? 0 : -5);
-            break;
         }
     }
     if (tid == 0) {
@@ -505,8 +357,34 @@ __device__ void team_solve(const BatchArgs &a, int sys, float *pan32, double *pa
     team_sync<TEAM>();
 }
 
-__global__ void batched_reset_kernel(unsigned *counter) { *counter = 0u; }
+__global__ void batched_reset_kernel(unsigned *counter) { counter[threadIdx.x] = 0u; }
 
+// FP64 launch: systems up to this size one per wave, larger ones by a whole workgroup
+// (NMAX / 4 is what a wave's slice of LDS holds; 4000 systems of 33 to 64 rows: 1.4 ms, by
+// workgroups 3.1; 8000 of 8 to 32: 0.86 and 1.9)
+constexpr int FP64_WAVE_MAX = NMAX / 4;
+constexpr int NEED_FP64 = -1000;     // status between the two launches
+
+// systems order[0..gridDim.x), all of one kind
+template <bool CHOL>
+__global__ __launch_bounds__(64, 2) void batched_wave_kernel(BatchArgs a, const int *order)
+{
+    extern __shared__ __align__(16) char wave_lds[];
+    const int sys = order[blockIdx.x];
+    const BatchDesc d = a.desc[sys];
+    int iters = 0;
+    double bwd = 0.0;
+    const bool ok = wave::solve<CHOL>(d.n, d.nrhs, a.A + d.offA, a.B + d.offB, a.X + d.offB, a.work + d.offW,
+                                      a.tol_scale * d.n * 0x1p-53, a.max_iter, wave_lds, threadIdx.x, &iters, &bwd);
+    if (threadIdx.x == 0) {
+        a.status[sys] = ok ? 0 : NEED_FP64;
+        a.iters[sys] = iters;
+        a.bwd[sys] = bwd;
+        if (!ok) __hip_atomic_store(a.counter + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// the systems that need FP64, one workgroup or wave each
 __global__ __launch_bounds__(NT) void batched_solve_kernel(BatchArgs a)
 {
     // one NMAX x (NB+1) FP64 panel for a whole-workgroup system, or four
@@ -514,11 +392,11 @@ __global__ __launch_bounds__(NT) void batched_solve_kernel(BatchArgs a)
     __shared__ double panbuf[NMAX * (NB + 1)];
     __shared__ double vec[4][2 * NMAX];
     __shared__ double red[8];
-    __shared__ float redf[8];
     __shared__ int redi[8];
     __shared__ int s_item;
     constexpr int SLICE = NMAX / 4 * (NB + 1);   // doubles per wave slice
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (a.counter[1] == 0u) return;
     while (true) {
         if (t == 0) s_item = (int)atomicAdd(a.counter, 4u);
         __syncthreads();
@@ -528,15 +406,17 @@ __global__ __launch_bounds__(NT) void batched_solve_kernel(BatchArgs a)
         for (int q = 0; q < 4 && item + q < a.batch; ++q) {
             const int sys = a.order[item + q];
             if (a.desc[sys].n > a.wave_max) {
-                team_solve<NT>(a, sys, reinterpret_cast<float *>(panbuf), panbuf, &vec[0][0], red, redf, redi, t);
+                const bool mine = a.status[sys] == NEED_FP64;
+                __syncthreads();   // read by every wave before the result is written
+                if (mine) team_solve<NT>(a, sys, panbuf, &vec[0][0], red, redi, t);
             } else {
                 // the remaining small entries of this pop: one per wave
                 const int qq = q + wave;
                 if (qq < 4 && item + qq < a.batch) {
                     const int s2 = a.order[item + qq];
-                    double *slice = panbuf + (size_t)wave * SLICE;
-                    team_solve<64>(a, s2, reinterpret_cast<float *>(slice), slice, vec[wave], red + 2 * wave,
-                                   redf + 2 * wave, redi + 2 * wave, lane);
+                    if (a.status[s2] == NEED_FP64)
+                        team_solve<64>(a, s2, panbuf + (size_t)wave * SLICE, vec[wave], red + 2 * wave, redi + 2 * wave,
+                                       lane);
                 }
                 __syncthreads();
                 break;
@@ -550,12 +430,10 @@ __global__ __launch_bounds__(NT) void batched_solve_kernel(BatchArgs a)
 // ===================================================================== host
 #include "api_internal.hpp"
 #include <string>
-int mkdir_p(const std::string &dir);
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <map>
 #include <string>
 #include <vector>
 
@@ -565,7 +443,8 @@ struct BatchPlan {
     uint64_t key = 0;
     int batch = 0;
     BatchDesc *d_desc = nullptr;
-    int *d_order = nullptr;
+    int *d_order = nullptr, *d_kinds = nullptr;   // by size; general systems by size, then SPD ones by size
+    int general = 0;
     long *d_offP = nullptr;
     int *d_status = nullptr, *d_iters = nullptr;
     double *d_bwd = nullptr;
@@ -576,65 +455,21 @@ struct BatchPlan {
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
     int graph_wave_max = -1;
-    std::string tune_key;
+    int nmax = 0;
 };
 
 BatchPlan g_plan;
-std::map<std::string, int> g_tune;      // size-histogram key -> wave_max
-bool g_tune_loaded = false;
-
-std::string tune_path()
-{
-    const char *p = getenv("SCIRS_GPU_TUNE_FILE");
-    if (p && *p) return p;
-    const char *h = getenv("HOME");
-    return std::string(h ? h : "/tmp") + "/.cache/scirs_gpu_batched_tune.json";
-}
-
-void tune_load()
-{
-    if (g_tune_loaded) return;
-    g_tune_loaded = true;
-    FILE *f = fopen(tune_path().c_str(), "r");
-    if (!f) return;
-    char key[256];
-    int v;
-    // the file is a flat JSON object {"key": value, ...}; read it token by token
-    int c;
-    while ((c = fgetc(f)) != EOF) {
-        if (c != '"') continue;
-        int k = 0;
-        while ((c = fgetc(f)) != EOF && c != '"' && k < 255) key[k++] = (char)c;
-        key[k] = 0;
-        while ((c = fgetc(f)) != EOF && c != ':') {}
-        if (fscanf(f, "%d", &v) == 1) g_tune[key] = v;
-    }
-    fclose(f);
-}
-
-void tune_save()
-{
-    std::string path = tune_path();
-    std::string dir = path.substr(0, path.find_last_of('/'));
-    if (!dir.empty()) {
-        (void)mkdir_p(dir);   // create the cache directory if needed
-    }
-    FILE *f = fopen(path.c_str(), "w");
-    if (!f) return;
-    fprintf(f, "{");
-    bool first = true;
-    for (auto &kv : g_tune) {
-        fprintf(f, "%s\"%s\": %d", first ? "" : ", ", kv.first.c_str(), kv.second);
-        first = false;
-    }
-    fprintf(f, "}\n");
-    fclose(f);
-}
-
+// FNV-1a over 8-byte words (a last partial word is padded with zeros)
 uint64_t fnv1a(uint64_t h, const void *p, size_t n)
 {
     const unsigned char *b = (const unsigned char *)p;
-    for (size_t i = 0; i < n; ++i) { h ^= b[i]; h *= 1099511628211ull; }
+    for (size_t i = 0; i < n; i += 8) {
+        uint64_t w = 0;
+        memcpy(&w, b + i, std::min<size_t>(8, n - i));
+        h ^= w;
+        h *= 1099511628211ull;
+        h ^= h >> 32;
+    }
     return h;
 }
 
@@ -664,28 +499,21 @@ int launch_batch(BatchPlan &pl, const double *dA, const double *dB, double *dX, 
     a.A = dA; a.B = dB; a.X = dX; a.work = pl.d_work; a.perm = pl.d_perm; a.offP = pl.d_offP;
     a.status = pl.d_status; a.iters = pl.d_iters; a.bwd = pl.d_bwd; a.counter = pl.d_counter;
     a.wave_max = wave_max; a.max_iter = max_iter; a.tol_scale = tol_scale;
-    hipLaunchKernelGGL(batched_reset_kernel, dim3(1), dim3(1), 0, s, pl.d_counter);
-    // a persistent grid: a few workgroups per CU pull work from the queue
-    const int grid = std::min(pl.batch, scirs::ctx().cu_count * 2);
-    hipLaunchKernelGGL(batched_solve_kernel, dim3(std::max(grid, 1)), dim3(NT), 0, s, a);
+    hipLaunchKernelGGL(batched_reset_kernel, dim3(1), dim3(2), 0, s, pl.d_counter);
+    if (pl.general)
+        hipLaunchKernelGGL(batched_wave_kernel<false>, dim3(pl.general), dim3(64), wave::lds_bytes(pl.nmax), s, a,
+                           pl.d_kinds);
+    if (pl.general < pl.batch)
+        hipLaunchKernelGGL(batched_wave_kernel<true>, dim3(pl.batch - pl.general), dim3(64), wave::lds_bytes(pl.nmax),
+                           s, a, pl.d_kinds + pl.general);
+    // a persistent grid: one workgroup per CU (LDS allows one) pulls work from the queue
+    const int grid = std::min(pl.batch, scirs::ctx().cu_count);
+    hipLaunchKernelGGL(batched_solve_kernel, dim3(grid), dim3(NT), 0, s, a);
     SCIRS_HIP_CHECK(hipGetLastError());
     return SCIRS_OK;
 }
 
 } // namespace
-
-static int mkdir_p_impl(const std::string &dir);
-int mkdir_p(const std::string &dir) { return mkdir_p_impl(dir); }
-#include <sys/stat.h>
-static int mkdir_p_impl(const std::string &dir)
-{
-    std::string cur;
-    for (size_t i = 0; i < dir.size(); ++i) {
-        cur += dir[i];
-        if (dir[i] == '/' || i + 1 == dir.size()) mkdir(cur.c_str(), 0755);
-    }
-    return 0;
-}
 
 extern "C" int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *nrhs, const unsigned char *spd,
                                            const double *dA, const int64_t *offA, const double *dB,
@@ -731,24 +559,27 @@ extern "C" int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *n
         std::vector<BatchDesc> desc(batch);
         std::vector<long> offP(batch);
         long work = 0, pw = 0;
-        long nsum = 0, nmax = 0;
+        int nmax = 0;
         for (int i = 0; i < batch; ++i) {
             desc[i].n = n[i]; desc[i].nrhs = nrhs[i]; desc[i].spd = spd ? spd[i] : 0; desc[i].pad = 0;
             desc[i].offA = offA[i]; desc[i].offB = offB[i]; desc[i].offW = work;
-            work += (long)n[i] * n[i];
+            work += std::max(((long)n[i] * n[i] + 15) & ~15L, wave::work_doubles(n[i]));
             offP[i] = pw; pw += n[i];
-            nsum += n[i]; nmax = std::max<long>(nmax, n[i]);
+            nmax = std::max(nmax, n[i]);
         }
         std::vector<int> order(batch);
         for (int i = 0; i < batch; ++i) order[i] = i;
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return n[x] > n[y]; });
+        std::vector<int> kinds(order);
+        pl.general = (int)(std::stable_partition(kinds.begin(), kinds.end(), [&](int x) { return !desc[x].spd; }) -
+                           kinds.begin());
         if ((rc = grow(&pl.d_desc, &pl.cap_batch, batch))) return rc;
-        size_t cap2 = 0, cap3 = 0, cap4 = 0, cap5 = 0, cap6 = 0;
+        size_t cap1 = 0, cap2 = 0, cap3 = 0, cap4 = 0, cap5 = 0, cap6 = 0;
         // the per-system arrays are (re)allocated together with the descriptors
-        if (pl.d_order) { (void)hipFree(pl.d_order); (void)hipFree(pl.d_offP); (void)hipFree(pl.d_status);
+        if (pl.d_order) { (void)hipFree(pl.d_order); (void)hipFree(pl.d_kinds); pl.d_kinds = nullptr; (void)hipFree(pl.d_offP); (void)hipFree(pl.d_status);
                           (void)hipFree(pl.d_iters); (void)hipFree(pl.d_bwd); pl.d_order = nullptr; pl.d_offP = nullptr;
                           pl.d_status = nullptr; pl.d_iters = nullptr; pl.d_bwd = nullptr; }
-        if ((rc = grow(&pl.d_order, &cap2, batch)) || (rc = grow(&pl.d_offP, &cap3, batch)) ||
+        if ((rc = grow(&pl.d_order, &cap2, batch)) || (rc = grow(&pl.d_kinds, &cap1, batch)) || (rc = grow(&pl.d_offP, &cap3, batch)) ||
             (rc = grow(&pl.d_status, &cap4, batch)) || (rc = grow(&pl.d_iters, &cap5, batch)) ||
             (rc = grow(&pl.d_bwd, &cap6, batch)))
             return rc;
@@ -760,48 +591,22 @@ extern "C" int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *n
         }
         SCIRS_HIP_CHECK(hipMemcpy(pl.d_desc, desc.data(), sizeof(BatchDesc) * batch, hipMemcpyHostToDevice));
         SCIRS_HIP_CHECK(hipMemcpy(pl.d_order, order.data(), sizeof(int) * batch, hipMemcpyHostToDevice));
+        SCIRS_HIP_CHECK(hipMemcpy(pl.d_kinds, kinds.data(), sizeof(int) * batch, hipMemcpyHostToDevice));
         SCIRS_HIP_CHECK(hipMemcpy(pl.d_offP, offP.data(), sizeof(long) * batch, hipMemcpyHostToDevice));
         if (pl.exec) { (void)hipGraphExecDestroy(pl.exec); pl.exec = nullptr; }
         if (pl.graph) { (void)hipGraphDestroy(pl.graph); pl.graph = nullptr; }
         pl.key = key;
         pl.batch = batch;
-        char tk[128];
-        snprintf(tk, sizeof(tk), "gfx950:nmax%ld:nmean%ld", (nmax + 31) / 32 * 32, (nsum / batch + 31) / 32 * 32);
-        pl.tune_key = tk;
+        pl.nmax = nmax;
     }
 
-    // ---- schedule crossover: explicit, tuned table, or tune now
-    int wave_max = -1;
+    // crossover of the FP64 launch; a wave's LDS slice holds systems up to NMAX / 4 rows
+    int wave_max = FP64_WAVE_MAX;
     const char *wm = getenv("SCIRS_GPU_BATCH_WAVE_MAX");
-    if (wm && *wm) wave_max = atoi(wm);
-    if (wave_max < 0) {
-        tune_load();
-        auto it = g_tune.find(pl.tune_key);
-        if (it != g_tune.end()) wave_max = it->second;
-    }
-    if (wave_max < 0) {
-        const int cand[3] = {0, 32, 64};
-        float best = 1e30f;
-        scirs::CallEvents ev;
-        if (int erc = ev.create(2)) return erc;
-        hipEvent_t e0 = ev.e[0], e1 = ev.e[1];
-        for (int ci = 0; ci < 3; ++ci) {
-            SCIRS_HIP_CHECK(hipEventRecord(e0, s));
-            if ((rc = launch_batch(pl, dA, dB, dX, cand[ci], max_iter, tol_scale, s))) return rc;
-            SCIRS_HIP_CHECK(hipEventRecord(e1, s));
-            SCIRS_HIP_CHECK(hipEventSynchronize(e1));
-            float ms = 0;
-            SCIRS_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-            if (ms < best) { best = ms; wave_max = cand[ci]; }
-        }
-        g_tune[pl.tune_key] = wave_max;
-        tune_save();
-    }
+    if (wm && *wm && atoi(wm) >= 0) wave_max = atoi(wm);
+    wave_max = std::min(wave_max, NMAX / 4);
 
-    // a wave's LDS slice holds systems up to NMAX / 4 rows
-    wave_max = std::max(0, std::min(wave_max, NMAX / 4));
-
-    // ---- one graph per plan and crossover: [reset queue, persistent solve], replayed
+    // ---- one graph per plan and crossover: [reset queue, FP32 solve, FP64 solve], replayed
     bool replay = true;
     if (!pl.exec || pl.graph_wave_max != wave_max) {
         replay = false;
