@@ -271,12 +271,12 @@ long round_up(long x, long m) { return (x + m - 1) / m * m; }
 // — one pass of partial products V^T C, one rank-32 product on the matrix
 // cores — instead of two passes per column.
 constexpr int QB = 32;        // panel width
-constexpr int PR = 256;       // rows per panel workgroup, one per thread
+constexpr int PR = 256;       // rows per panel workgroup (and its threads)
 constexpr int QG_MAX = 64;    // panel workgroups: rows - k0 <= QG_MAX * PR
 constexpr int QKC = 32;       // row chunks of the partial products V^T C (at most)
 constexpr int QWT = 256;      // columns per partial-product workgroup
 typedef unsigned long long u64;
-constexpr size_t QXW_WORDS = 2ull * QG_MAX * (QB + 1) * 2;   // exchange words (2 per value)
+constexpr size_t QXW_WORDS = 2ull * (QG_MAX + 1) * QB * 2;   // exchange words (2 per value)
 
 __device__ __forceinline__ void qx_put(u64 *w, unsigned seq, double v)
 {
@@ -291,142 +291,184 @@ __device__ __forceinline__ bool qx_get(const u64 *w, unsigned seq, double &v)
     v = __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
     return (unsigned)(lo >> 32) == seq && (unsigned)(hi >> 32) == seq;
 }
-// poll one tagged value; false when the wait gave up (or another workgroup did)
-__device__ bool qx_wait(const u64 *w, unsigned seq, double &v, unsigned spin_limit, int *abort)
-{
-    for (unsigned it = 0;; ++it) {
-        if (qx_get(w, seq, v)) return true;
-        if (it >= spin_limit || __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-            __hip_atomic_store(abort, (int)SCIRS_ABORT_QR_PANEL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
-        __builtin_amdgcn_s_sleep(1);
-    }
-}
-
 struct QPanelArgs {
     double *R; long ldr;
     int rows, k0, w, G;
     double *V;          // rows x QB, ld QB: the panel's reflectors (0 above their first row, 0 past w)
     int *flags;         // [QB]: 1 reflector applied, 0 column skipped
-    u64 *xw;            // [2][QG_MAX][QB + 1][2]: phase 0 (sums of squares, x0), phase 1 (dots)
-    unsigned seq;       // phase p of column j uses seq + 2 j + p
+    u64 *xw;            // [column parity][pivot row, QG_MAX workgroups' sums][QB][2]
+    unsigned seq;       // column j uses seq + j
     int *abort; unsigned spin_limit;
 };
 
-// The reflectors of columns k0 .. k0 + w - 1 with the reference's arithmetic
-// (lapack.rs:205-235): per column the sum of squares, alpha = -sign(x0) ||x||,
-// v = (x - alpha e1) / ||v||, and H = I - 2 v v^T on the panel's columns
-// j.. .  G workgroups hold PR rows each in LDS; the two sums a column needs
-// (||x||^2 and the dots v^T a_c) are exchanged as sequence-tagged words and
-// added in workgroup order, so every workgroup computes the same alpha and v.
-// The exchanged sum covers the rows below the pivot row, so ||x||^2 = x0^2 +
-// tail and ||v||^2 = (x0 - alpha)^2 + tail (as the reference sums v_i^2, v0
-// first) come from one exchange without cancellation.
+// sum over the lanes of a wave that hold the same columns (lane bits 3, 4 and 5), to all of them
+__device__ __forceinline__ double sum_row_lanes(double v)
+{
+    auto add = [](double x, auto swap) {
+        const u64 b = (u64)__double_as_longlong(x);
+        const auto lo = swap((unsigned)b), hi = swap((unsigned)(b >> 32));
+        return __longlong_as_double((long long)(((u64)hi[0] << 32) | lo[0])) +
+               __longlong_as_double((long long)(((u64)hi[1] << 32) | lo[1]));
+    };
+    v += dpp_val<0x128, 0xf>(0.0, v);   // row_ror:8
+    v = add(v, [](unsigned x) { return __builtin_amdgcn_permlane16_swap(x, x, false, false); });
+    return add(v, [](unsigned x) { return __builtin_amdgcn_permlane32_swap(x, x, false, false); });
+}
+
+// The reflectors of columns k0 .. k0 + w - 1 (lapack.rs:205-235): per column
+// alpha = -sign(x0) ||x||, v = (x - alpha e1) / ||v||, and H = I - 2 v v^T on
+// the panel's columns j.. .  G workgroups hold PR rows each in registers,
+// thread (c4, rg) the columns 4 c4 .. 4 c4 + 3 of the rows rg, rg + 32, ... .
+//
+// A column is bound by its exchange between workgroups, so there is one: the
+// sums S_c = x^T a_c over the rows below the pivot row, for every column c of
+// the panel, and the pivot row itself.  S_j is the tail of ||x||^2 = x0^2 + S_j
+// and of ||v||^2 = (x0 - alpha)^2 + S_j (no cancellation), and v^T a_c =
+// ((x0 - alpha) a_rj,c + S_c) / ||v||.  The words are tagged with the column's
+// sequence number; two copies alternate, since a workgroup may publish column
+// j + 1 while another still reads column j (j + 2 needs everyone's j + 1).  The
+// sums are added in workgroup order: every workgroup gets the same alpha and v.
+// 8192 rows: 152 us per panel of 32 columns; 234 with two exchanges per column
+// (the norm, then the dots), the panel in LDS and polls one after the other.
 __global__ __launch_bounds__(PR) void qr_panel_kernel(QPanelArgs a)
 {
     // products rounded before they are added, as in the reference's loops
 #pragma clang fp contract(off)
-    __shared__ double P[PR][QB + 1];
-    __shared__ double xd[QG_MAX][QB];
-    __shared__ double red[PR / 32][QB];
-    __shared__ double vcol[PR];
-    __shared__ double tot[QB + 1];
+    constexpr int M = PR / 32;                  // rows per thread
+    __shared__ double Vs[PR][QB + 1];
+    __shared__ double xcol[2][PR];
+    __shared__ __align__(16) double red[PR / 64][QB], sums[PR / 32][QB], prow[QB];
     __shared__ int s_fail;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, g = blockIdx.x;
-    const int row = a.k0 + g * PR + t;
-    const bool have = row < a.rows;
-    for (int c = 0; c < QB; ++c) P[t][c] = (have && c < a.w) ? a.R[(long)row * a.ldr + a.k0 + c] : 0.0;
+    const int c4 = t & 7, rg = t >> 3, gs = t >> 5, cq = t & (QB - 1);
+    const int r0 = a.k0 + g * PR + rg;          // row of m = 0
+    double p[M][4];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        const double *src = a.R + (long)(r0 + 32 * m) * a.ldr + a.k0 + 4 * c4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) p[m][q] = r0 + 32 * m < a.rows && 4 * c4 + q < a.w ? src[q] : 0.0;
+    }
+    if (c4 == 0)
+#pragma unroll
+        for (int m = 0; m < M; ++m) xcol[0][rg + 32 * m] = p[m][0];
     if (t == 0) s_fail = 0;
     __syncthreads();
-    u64 *x0w = a.xw, *x1w = a.xw + (size_t)QG_MAX * (QB + 1) * 2;
-    for (int j = 0; j < a.w; ++j) {
-        const int rj = a.k0 + j;
-        const unsigned sq0 = a.seq + 2u * j, sq1 = sq0 + 1u;
-        // (a) this workgroup's sum of squares of column j below the pivot row
-        //     (rows > rj); the pivot row rj lies in workgroup 0, which also
-        //     publishes x0
-        const double x = (have && row >= rj) ? P[t][j] : 0.0;
-        const double ws = wave_sum(row > rj ? x * x : 0.0);
-        if (lane == 0) red[wave][0] = ws;
-        __syncthreads();
-        if (t == 0) {
-            double ss = 0.0;
-            for (int q = 0; q < PR / 64; ++q) ss += red[q][0];
-            qx_put(x0w + ((size_t)g * (QB + 1)) * 2, sq0, ss);
-            qx_put(x0w + ((size_t)g * (QB + 1) + 1) * 2, sq0, g == 0 ? P[j][j] : 0.0);
-        }
-        if (wave == 0) {
-            double v = 0.0;
-            bool ok = true;
-            if (lane < a.G) ok = qx_wait(x0w + ((size_t)lane * (QB + 1)) * 2, sq0, v, a.spin_limit, a.abort);
-            double x0 = 0.0;
-            if (lane == 0 && ok) ok = qx_wait(x0w + 2, sq0, x0, a.spin_limit, a.abort);
-            const double sum = wave_sum(v);
-            if (!ok) s_fail = 1;
-            if (lane == 0) {
-                tot[0] = sum;
-                tot[1] = x0;
+    for (int j4 = 0; 4 * j4 < a.w; ++j4) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = 4 * j4 + e;
+            if (j >= a.w) break;
+            const int rj = a.k0 + j;
+            const unsigned seq = a.seq + j;
+            u64 *pw = a.xw + (size_t)(e & 1) * (QG_MAX + 1) * QB * 2, *sw = pw + QB * 2;
+            // this workgroup's sums, and the pivot row (row j of workgroup 0)
+            double x[M], s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                x[m] = r0 + 32 * m >= rj ? xcol[e & 1][rg + 32 * m] : 0.0;
+                const double below = r0 + 32 * m > rj ? x[m] : 0.0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s[q] += below * p[m][q];
             }
-        }
-        __syncthreads();
-        if (s_fail) return;
-        const double tail = tot[0], x0 = tot[1];
-        const double xn = sqrt(x0 * x0 + tail);
-        bool apply = xn > DBL_EPSILON;
-        double alpha = 0.0, v0 = 0.0, vn = 1.0;
-        if (apply) {
-            alpha = x0 >= 0.0 ? -xn : xn;
-            v0 = x0 - alpha;
-            vn = sqrt(v0 * v0 + tail);
-            apply = vn > DBL_EPSILON;
-        }
-        if (g == 0 && t == 0) a.flags[j] = apply ? 1 : 0;
-        const double vi = (!apply || !have || row < rj) ? 0.0 : (row == rj ? v0 / vn : x / vn);
-        if (have) a.V[(long)row * QB + j] = vi;
-        if (!apply) continue;   // the same decision in every workgroup
-        vcol[t] = vi;
-        __syncthreads();
-        // (b) dots d_c = v^T a_c for the panel's columns c >= j: 32 columns x
-        //     8 row groups, the groups added in order, then exchanged
-        {
-            const int cc = t & (QB - 1), rg = t >> 5;
-            double d = 0.0;
-            if (cc >= j && cc < a.w)
-                for (int i = rg; i < PR; i += PR / 32) d += vcol[i] * P[i][cc];
-            red[rg][cc] = d;
-        }
-        __syncthreads();
-        if (t < QB && t >= j && t < a.w) {
-            double d = 0.0;
-            for (int q = 0; q < PR / 32; ++q) d += red[q][t];
-            qx_put(x1w + ((size_t)g * (QB + 1) + t) * 2, sq1, d);
-        }
-        for (int q = t; q < a.G * QB; q += PR) {
-            const int gq = q / QB, cq = q % QB;
-            if (cq >= j && cq < a.w) {
-                double v;
-                if (!qx_wait(x1w + ((size_t)gq * (QB + 1) + cq) * 2, sq1, v, a.spin_limit, a.abort)) s_fail = 1;
-                xd[gq][cq] = v;
+            if (g == 0 && rg == j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) qx_put(pw + (4 * c4 + q) * 2, seq, p[0][q]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) s[q] = sum_row_lanes(s[q]);
+            if (lane < 8)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) red[wave][4 * lane + q] = s[q];
+            __syncthreads();
+            if (t < QB) qx_put(sw + ((size_t)g * QB + t) * 2, seq, (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]));
+            // everyone's sums of column cq: workgroups gs, gs + 8, ..., all loads in flight together
+            {
+                double v[QG_MAX / 8], pv = 0.0;
+                for (unsigned it = 0;; ++it) {
+                    bool ok = true;
+#pragma unroll
+                    for (int u = 0; u < QG_MAX / 8; ++u) {
+                        v[u] = 0.0;
+                        if (gs + 8 * u < a.G) ok &= qx_get(sw + ((size_t)(gs + 8 * u) * QB + cq) * 2, seq, v[u]);
+                    }
+                    if (gs == 0) ok &= qx_get(pw + cq * 2, seq, pv);
+                    if (ok) break;
+                    if (it >= a.spin_limit || __hip_atomic_load(a.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+                        __hip_atomic_store(a.abort, (int)SCIRS_ABORT_QR_PANEL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        s_fail = 1;
+                        break;
+                    }
+                }
+                double sum = 0.0;
+#pragma unroll
+                for (int u = 0; u < QG_MAX / 8; ++u) sum += v[u];
+                sums[gs][cq] = sum;
+                if (gs == 0) prow[cq] = pv;
             }
+            __syncthreads();
+            if (s_fail) return;
+            double tail = 0.0, f[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int u = 0; u < PR / 32; ++u) {
+                tail += sums[u][j];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) f[q] += sums[u][4 * c4 + q];
+            }
+            const double x0 = prow[j], xn = sqrt(x0 * x0 + tail);
+            bool apply = xn > DBL_EPSILON;
+            double v0 = 0.0, vn = 1.0;
+            if (apply) {
+                v0 = x0 - (x0 >= 0.0 ? -xn : xn);
+                vn = sqrt(v0 * v0 + tail);
+                apply = vn > DBL_EPSILON;
+            }
+            if (g == 0 && t == 0) a.flags[j] = apply ? 1 : 0;
+            // x / vn by the reciprocal and one residual correction
+            double rv = __builtin_amdgcn_rcp(vn);
+            rv = fma(rv, fma(-vn, rv, 1.0), rv);
+            rv = fma(rv, fma(-vn, rv, 1.0), rv);
+            auto over_vn = [&](double n) {
+                const double q = n * rv;
+                return fma(fma(-q, vn, n), rv, q);
+            };
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int row = r0 + 32 * m;
+                x[m] = apply ? over_vn(row == rj ? v0 : x[m]) : 0.0;
+                if (c4 == (j & 7)) Vs[rg + 32 * m][j] = x[m];
+            }
+            // H on the columns from j on (the finished ones stay)
+            if (apply) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) f[q] = 2.0 * over_vn(v0 * prow[4 * c4 + q] + f[q]);
+                if (c4 > j4) {
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) p[m][q] -= x[m] * f[q];
+                } else if (c4 == j4) {
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+#pragma unroll
+                        for (int q = e; q < 4; ++q) p[m][q] -= x[m] * f[q];
+                }
+            }
+            if (c4 == j4 + (e == 3))
+#pragma unroll
+                for (int m = 0; m < M; ++m) xcol[(e + 1) & 1][rg + 32 * m] = p[m][(e + 1) & 3];
+            __syncthreads();
         }
-        __syncthreads();
-        if (s_fail) return;
-        if (t < QB && t >= j && t < a.w) {
-            double d = 0.0;
-            for (int q = 0; q < a.G; ++q) d += xd[q][t];
-            tot[t] = d;
-        }
-        __syncthreads();
-        // (c) H on this workgroup's rows of columns j.. (the reference's
-        //     r_ic -= 2 v_i (v^T c))
-        if (have)
-            for (int c = j; c < a.w; ++c) P[t][c] -= 2.0 * vi * tot[c];
-        __syncthreads();
     }
-    if (have) {
-        for (int c = 0; c < a.w; ++c) a.R[(long)row * a.ldr + a.k0 + c] = P[t][c];
-        for (int c = a.w; c < QB; ++c) a.V[(long)row * QB + c] = 0.0;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        double *dst = a.R + (long)(r0 + 32 * m) * a.ldr + a.k0 + 4 * c4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (r0 + 32 * m < a.rows && 4 * c4 + q < a.w) dst[q] = p[m][q];
+    }
+    for (int i = t; i < PR * QB; i += PR) {
+        const int r = i / QB, c = i % QB, row = a.k0 + g * PR + r;
+        if (row < a.rows) a.V[(long)row * QB + c] = c < a.w ? Vs[r][c] : 0.0;
     }
 }
 
@@ -613,7 +655,7 @@ int householder_blocked(int rows, int cols, int rcols, double *R, long ldr, doub
     q.flags = (int *)(q.Y + (size_t)QB * ldp);
     for (int k0 = 0; k0 < kmax; k0 += QB) {
         const int w = std::min(QB, kmax - k0), rows_k = rows - k0;
-        if (q.seq > 0xFFFFFFFFu - 2u * QB) {
+        if (q.seq > 0xFFFFFFFFu - QB) {
             fill_u64_kernel<<<(unsigned)((QXW_WORDS + 255) / 256), 256, 0, s>>>(q.xw, QXW_WORDS);
             q.seq = 1;
         }
@@ -622,7 +664,7 @@ int householder_blocked(int rows, int cols, int rcols, double *R, long ldr, doub
         pa.G = (rows_k + PR - 1) / PR;
         pa.V = q.V; pa.flags = q.flags; pa.xw = q.xw; pa.seq = q.seq;
         pa.abort = c.work.abort; pa.spin_limit = c.work.spin_limit;
-        q.seq += 2u * QB;
+        q.seq += QB;
         qr_panel_kernel<<<pa.G, PR, 0, s>>>(pa);
         const int rc0 = k0 + w, nR = rcols - rc0, ntot = QB + nR + nQ;
         // enough row chunks for about 512 workgroups, no more (every chunk adds
