@@ -351,7 +351,7 @@ __global__ __launch_bounds__(NTHREADS, OCC) void dgemm_fold_kernel(GemmArgs<doub
 
 // C (M x N) -= A B^T with K = 128 in 64 x 64 tiles, operands straight from L2 into the
 // matrix-core layout: small updates, whose 128 x 128 tiles would leave most CUs idle
-// and take 27 us a tile (8 us a tile here; the large tiles reuse their operands twice
+// and take 27 us a tile (9 to 11 us a launch here; the large tiles reuse their operands twice
 // as often and win once they fill the device).  lower: only tiles that touch C's lower
 // triangle.  k-order as above.
 struct Syrk64Args {

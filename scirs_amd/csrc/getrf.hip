@@ -2,13 +2,13 @@
 //
 // Algorithm (row-major A, the layout of an ndarray in standard order), per
 // panel of kb columns starting at k0:
-//   1. getf2_panel  — cooperative kernel.  The panel's m-k0 rows are split
-//      into contiguous chunks, one per workgroup, and kept in LDS for the whole
-//      panel.  Each column: wave64 arg-max over the chunk, candidates published
-//      to global memory, one grid barrier, every workgroup reduces the same
-//      candidate list (lowest row wins ties, the strict '>' scan of
-//      scirs2-linalg/src/lapack.rs:95-104), swaps, divides and applies the
-//      rank-1 update to its own rows.  The absolute singularity test of
+//   1. panel        — sub-panels of 32 columns with rows in registers
+//      (sub_panel_kernel, subpanel.hip), each followed by one launch that
+//      interchanges, solves U12 and updates (sub_apply_kernel): the whole rest
+//      of the matrix up to LU_SINGLE rows, the panel's later columns above.
+//      Taller panels than the registers hold run in getf2_panel (panel.hpp).
+//      The pivot is the first maximum (the strict '>' scan of
+//      scirs2-linalg/src/lapack.rs:95-104); the absolute singularity test of
 //      lapack.rs:106-120 (|pivot| < eps) stops the factorisation with
 //      info = column + 1.
 //   2. laswp        — applies the panel's net row permutation to the columns
@@ -16,7 +16,7 @@
 //   3. trsm         — U12 = L11^-1 A12: FP64 by substitution in 64-column strips
 //      with L11 (packed) and the strip in LDS; FP32 by forming L11^-1 in one
 //      workgroup and multiplying the strips by it.
-//   4. dgemm        — A22 -= L21 U12 on the matrix cores (gemm_f64.hip).
+//   4. dgemm        — A22 -= L21 U12 on the matrix cores (gemm_mfma.hip).
 //
 // The arithmetic per element is the reference's (multiplier by true division,
 // a_ij -= l_ik * u_kj); only the order of the k-sum differs (blocked), which
@@ -37,7 +37,6 @@ constexpr int NT = 256;  // threads per workgroup everywhere in this file
 // rows up to which the LU runs in single 32-column sub-panels, each followed by
 // the update of every column right of it
 constexpr int LU_SINGLE_F64 = 2048, LU_SINGLE_F32 = 2048;
-
 
 // Apply a gather list to nv columns: the first nleft are columns 0..nleft-1,
 // the others start at column right0.  Each workgroup owns 64 columns, stages

@@ -4,7 +4,8 @@
 // (`iterative_refinement_solve`), which re-factors A in the working precision
 // on every step and stops on an absolute residual.  Here:
 //   1. A32 = fp32(A) fused with the row sums of |A| (||A||_inf);
-//   2. LU of A32: FP32 panel with tournament pivoting, trailing update in the
+//   2. LU of A32: FP32 register panels with partial pivoting (tournament pivoting
+//      for panels taller than the registers hold), trailing update in the
 //      requested arithmetic (BF16 / FP16-scaled / split-BF16 / split-FP16 /
 //      FP32 matrix cores, FP32 accumulation);
 //   3. refinement  R = B - A X (FP64, GPU), D = U^-1 L^-1 P R (FP32),

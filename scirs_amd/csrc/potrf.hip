@@ -44,9 +44,9 @@ __device__ __forceinline__ double readlane_t<double>(double v, int k)
 // waves exchange their L through LDS and update their later columns, which wait in
 // registers in the matrix-core layout.  The last workgroup to have read the diagonal
 // block (an arrival count, nobody waits) writes it back.
-// Bound by the column chain (about 400 cycles a column).  Measured for one 128-column
-// panel: 36 us whatever the rows below (up to one workgroup per CU), against
-// 78 (diagonal block) + 36 (its inverse) + 23 us (product) in three launches before.
+// Bound by the column chain.  Measured for one FP64 128-column panel: 45 to 50 us
+// whatever the rows below (up to one workgroup per CU), against 78 (diagonal block) + 36
+// (its inverse) + 23 us (product) in three launches before.
 // One a_jj - sum <= 0 sets info = row + 1 and stops.
 template <typename T> struct CholPanelArgs {
     T *A; long lda;

@@ -620,7 +620,7 @@ constexpr int ANT = 256, SC = 64, SP = SC + 2;   // threads, columns of a strip,
 // workgroups to have read those rows (an arrival count, nobody waits) writes the top
 // rows and the rows that the interchanges displaced, so no row is overwritten while
 // another workgroup may still read it.  Rank 32 per pass: latency-bound at small
-// sizes (about 8 us a launch), HBM-bound above.
+// sizes (12 to 20 us a launch for FP64 of up to 7000 rows), HBM-bound above.
 // A: the matrix; L11: the sub-panel's diagonal block (in columns that no workgroup writes).
 template <typename T>
 __global__ __launch_bounds__(ANT) void sub_apply_kernel(T *__restrict__ A, const T *__restrict__ L11, ApplyArgs<T> a)
