@@ -556,6 +556,8 @@ extern "C" int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *n
     key = fnv1a(key, &tol_scale, sizeof(tol_scale));
     const bool same = (pl.key == key && pl.batch == batch);
     if (!same) {
+        pl.key = 0;       // no plan until this one is complete
+        pl.batch = 0;
         std::vector<BatchDesc> desc(batch);
         std::vector<long> offP(batch);
         long work = 0, pw = 0;
