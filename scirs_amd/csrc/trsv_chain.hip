@@ -154,8 +154,11 @@ __device__ __forceinline__ void stage_tile(T *dst, const T *src, long ld, int ro
     }
 }
 
+// With several right-hand sides per chain, at most 256 registers: two workgroups per CU,
+// so that four chains of 128 links run side by side instead of two (FP64 Cholesky solve
+// n = 8192, 16 right-hand sides: 15.7 -> 15.3 ms).
 template <typename T, int QB, bool LOWER, bool UNIT>
-__global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A, long lda, T *X, long ldx, int n,
+__global__ __launch_bounds__(NTC, QB == 1 ? 1 : 2) void trsv_chain_kernel(const T *__restrict__ A, long lda, T *X, long ldx, int n,
                                                          int nrhs, u64 *xch, unsigned seq, int *ticket, int *abort,
                                                          unsigned spin_limit, int *info,
                                                          const T *__restrict__ dinv, const T *__restrict__ dmt)
@@ -194,14 +197,19 @@ __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A
         for (int j = wave - 1; j < b - 1; j += 3) {
             const int cb = LOWER ? j : nblk - 1 - j;
             const int c0 = cb * TB;
-            T a[16][4];
+            // a tile in NH parts: what a lane holds of it at a time fits the registers
+            constexpr int NH = sizeof(T) == 8 && QB > 1 ? 2 : 1, MH = 16 / NH;
+            T a[MH][4];
+            auto load_part = [&](int h) {
 #pragma unroll
-            for (int m = 0; m < 16; ++m) {
-                const int row = 4 * m + g;
-                const T *src = A + (long)(r0 + row) * lda + c0 + c;
+                for (int m = 0; m < MH; ++m) {
+                    const int row = 4 * (MH * h + m) + g;
+                    const T *src = A + (long)(r0 + row) * lda + c0 + c;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) a[m][e] = (row < bs && c0 + c + e < n) ? src[e] : (T)0;
-            }
+                    for (int e = 0; e < 4; ++e) a[m][e] = (row < bs && c0 + c + e < n) ? src[e] : (T)0;
+                }
+            };
+            load_part(0);
             T xv[4][QB];
             bool ok = true;
 #pragma unroll
@@ -212,11 +220,18 @@ __global__ __launch_bounds__(NTC) void trsv_chain_kernel(const T *__restrict__ A
             }
             if (!ok) { failed = true; break; }
 #pragma unroll
-            for (int m = 0; m < 16; ++m)
+            for (int h = 0; h < NH; ++h) {
+                if (h > 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load_part(h);
+                }
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
+                for (int m = 0; m < MH; ++m)
 #pragma unroll
-                    for (int q = 0; q < QB; ++q) acc[m][q] += a[m][e] * xv[e][q];
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int q = 0; q < QB; ++q) acc[MH * h + m][q] += a[m][e] * xv[e][q];
+            }
         }
         // reduce over the 16 lanes that share a row; lane (m) of each group keeps row 4m+g
 #pragma unroll
