@@ -4,7 +4,7 @@
 // What bounds it: a small system is a chain of short dependent steps (one per column of
 // the factor, one per 16 rows of each substitution), so the chip is filled with many
 // systems rather than one system with many threads.  A wave needs no barrier and no
-// exchange through LDS between steps, and nine or more waves per CU cover each other's
+// exchange through LDS between steps, and eight waves per CU cover each other's
 // waits.  Everything else is arranged in 16 x 16 blocks for the matrix cores:
 //   - the factor runs over panels of 16 columns held in registers, one row per lane and
 //     64 rows per register set; the pivot row is broadcast through scalar registers and

@@ -2,7 +2,7 @@
 // of a row-major matrix, in ONE launch.
 //
 // Same arithmetic as the substitution loops of scirs2-linalg/src/solve.rs:159-199
-// (true division by the diagonal in FP64; multiplication by the reciprocal in
+// (the correctly rounded quotient in FP64; multiplication by the reciprocal in
 // FP32), with the k-sum split into 64-column blocks.  The matrix is cut into 64-row block rows; block row p is solved by one
 // workgroup once the x values of every block it depends on are known.
 //
