@@ -154,7 +154,7 @@ int Context::init(int dev)
                  tpm_b = (2 * (size_t)TSLU_MAP + 1) * sizeof(int);
     const size_t sk_b = 2 * (size_t)SCIRS_SUB_AGENTS * 2 * 8, sr_b = 2 * (size_t)SCIRS_SUB_AGENTS * SCIRS_SUB_W * 2 * 8,
                  sc_b = (size_t)SCIRS_SUB_MAX * SCIRS_SUB_CTL * 4, sp_b = (size_t)SCIRS_SUB_MAX * SCIRS_SUB_PAIRS * 2 * 4,
-                 sa_b = (size_t)SCIRS_SUB_STRIPS * 4, sl_b = (size_t)SCIRS_SUB_ROWS * 4;
+                 sa_b = ((size_t)SCIRS_SUB_STRIPS + 1) * 4, sl_b = (size_t)SCIRS_SUB_ROWS * 4;
     for (size_t b : {sk_b, sr_b, sc_b, sp_b, sa_b, sl_b}) bytes += (b + 255) & ~(size_t)255;
     for (size_t b : {xw_b, xrow_b, xrj_b, flags_b, pairs_b, npairs_b, linv_b, tpc_b, tpn_b, tpu_b, tpr_b, tpt_b, tpt_b,
                      tpv_b, tpm_b})
@@ -191,6 +191,7 @@ int Context::init(int dev)
     work.sub_ctl = (int *)take(sc_b);
     work.sub_pairs = (int *)take(sp_b);
     work.sub_arrive = (int *)take(sa_b);
+    work.chol_arrive = work.sub_arrive + SCIRS_SUB_STRIPS;
     work.sub_label = (int *)take(sl_b);
     {
         std::vector<int> identity(SCIRS_SUB_ROWS);

@@ -55,6 +55,7 @@ struct ScirsWork {
     int *sub_ctl;                  // [SCIRS_SUB_MAX][SCIRS_SUB_CTL] election of the die, count of moved rows
     int *sub_pairs;                // [SCIRS_SUB_MAX][SCIRS_SUB_PAIRS][2] moved rows of a sub-panel
     int *sub_arrive;               // [SCIRS_SUB_STRIPS] arrival counts (zero between launches)
+    int *chol_arrive;              // arrival count of the Cholesky panel (zero between launches)
     int *sub_label;                // [SCIRS_SUB_ROWS] the identity between launches
 };
 

@@ -6,6 +6,7 @@
 //      launch; the reference's test `a_ii - sum <= 0` (lapack.rs:661-670) sets
 //      info = row + 1 and stops.
 //   2. syrk — A22 -= L21 L21^T on the matrix cores (lower tiles only).
+#include "arrive.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
 #include "lanes.hpp"
@@ -47,12 +48,20 @@ __device__ __forceinline__ double readlane_t<double>(double v, int k)
 // Bound by the column chain.  Measured for one FP64 128-column panel: 45 to 50 us
 // whatever the rows below (up to one workgroup per CU), against 78 (diagonal block) + 36
 // (its inverse) + 23 us (product) in three launches before.
-// One a_jj - sum <= 0 sets info = row + 1 and stops.
+// One a_jj - sum <= 0 sets info = row + 1 and stops; a workgroup that starts after that
+// still registers its arrival (arrive.hpp) before it leaves.
 template <typename T> struct CholPanelArgs {
     T *A; long lda;
     int k0, kb, n;
     int *arrive;      // zero between launches
     int *info; double *info_val;
+};
+struct CholArrival {
+    int *count;
+    bool failed;   // info as it was when the workgroup started
+    __device__ int add() { return __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ void clear() { __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ bool stopped() const { return failed; }
 };
 // x's lanes 0..15 (lo) and 16..31 (hi) in every row of 16 lanes
 __device__ __forceinline__ void spread(unsigned x, unsigned &lo, unsigned &hi)
@@ -140,15 +149,16 @@ template <typename T, int J> __device__ __forceinline__ int chol_columns(T (&a)[
 
 template <typename T> __global__ __launch_bounds__(NT, 2) void chol_panel_kernel(CholPanelArgs<T> g)
 {
-    if (*g.info != 0) return;
     using lanes::Mf;
     typedef typename Mf<T>::V V4;
     typedef typename lanes::Vec16<T>::type V;
     typedef typename lanes::Vec16u<T>::type Vu;
     constexpr int B = CP_B, E = 16 / (int)sizeof(T), P = B + E;   // LDS pitch: 16-byte rows
     __shared__ __align__(16) T Ls[5][B * P];   // the waves' row groups; [4]: the diagonal rows
-    __shared__ int s_last, s_fail;
+    __shared__ int s_last, s_stop, s_fail;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // read once, by one thread: workgroup 0 of this very launch may be setting it
+    const int info = t == 0 ? __hip_atomic_load(g.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
     const int l16 = lane & 15, grp = lane >> 4, l32 = lane & 31;
     const bool low = lane < 32;
     T *D = g.A + (long)g.k0 * g.lda + g.k0;
@@ -198,17 +208,16 @@ template <typename T> __global__ __launch_bounds__(NT, 2) void chol_panel_kernel
                         C[b][i][j][q] = ok ? v : (T)(wave < 3 && r == c ? 1 : 0);
                     }
     __builtin_amdgcn_s_waitcnt(0);
-    if (t == 0) s_fail = 0;
+    if (t == 0) {
+        s_fail = 0;
+        s_stop = info != 0;
+    }
     __syncthreads();
     if (t == 0) {
-        int last = 1;
-        if (gridDim.x > 1) {
-            last = __hip_atomic_fetch_add(g.arrive, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                   (int)gridDim.x - 1;
-            if (last) __hip_atomic_store(g.arrive, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        s_last = last;
+        CholArrival m{g.arrive, info != 0};
+        s_last = arrive::enter(m, (int)gridDim.x).last;
     }
+    if (s_stop) return;
 #pragma unroll
     for (int jb = 0; jb < 4; ++jb) {
         if (B * jb >= g.kb) break;
@@ -343,7 +352,7 @@ int scirs_potrf_device(int n, T *A, long lda, int kb, ScirsWork &w, hipStream_t 
         const int rest = n - k0 - kbw;
         CholPanelArgs<T> pa;
         pa.A = A; pa.lda = lda; pa.k0 = k0; pa.kb = kbw; pa.n = n;
-        pa.arrive = w.sub_arrive; pa.info = w.info; pa.info_val = w.info_val;
+        pa.arrive = w.chol_arrive; pa.info = w.info; pa.info_val = w.info_val;
         hipLaunchKernelGGL(chol_panel_kernel<T>, dim3(std::max(1, (rest + CP_B - 1) / CP_B)), dim3(NT), 0,
                            stream, pa);
         SCIRS_HIP_CHECK(hipGetLastError());
