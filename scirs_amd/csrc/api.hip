@@ -601,8 +601,8 @@ static int posv_device(int n, int nrhs, const T *dA, long lda, const T *dB, long
         T *dU = (T *)c.scratch_t;
         if ((rc = scirs_transpose_lower<T>(n, dL, ldl, dU, n, s))) return rc;
         if ((rc = c.ensure_xtri(n))) return rc;
-        if ((rc = scirs_trsv_chain<T>(n, nrhs, dL, ldl, dX, ldx, 1, 0, c.work, s))) return rc;
-        if ((rc = scirs_trsv_chain<T>(n, nrhs, dU, n, dX, ldx, 0, 0, c.work, s))) return rc;
+        if ((rc = scirs_trsv_chain<T>(n, nrhs, dL, ldl, dX, ldx, 1, 0, c.work, s, nullptr, nullptr, 1))) return rc;
+        if ((rc = scirs_trsv_chain<T>(n, nrhs, dU, n, dX, ldx, 0, 0, c.work, s, nullptr, nullptr, 1))) return rc;
     } else if ((rc = scirs_potrs_device<T>(n, nrhs, dL, ldl, dX, ldx, c.work.info, s))) {
         return rc;
     }

@@ -158,9 +158,11 @@ int scirs_trsv_big(int n, int nrhs, const T *A, long lda, T *X, long ldx, int lo
 // dmt (optional, with dinv): Dinv[p] times the tile block row p meets last
 // (scirs_tri_block_coupling, depth 3: a one-rhs FP32 solve then hands over
 // two block rows per link, using the couplings two and three blocks back)
+// halves: the last block's products in two sums instead of in column order; for
+// triangles that no pivoting made (Cholesky, QR)
 template <typename T>
 int scirs_trsv_chain(int n, int nrhs, const T *A, long lda, T *X, long ldx, int lower, int unit, ScirsWork &w,
-                     hipStream_t s, const T *dinv = nullptr, const T *dmt = nullptr);
+                     hipStream_t s, const T *dinv = nullptr, const T *dmt = nullptr, int halves = 0);
 
 // M_d[p] = Dinv[p] * (block row p's d-th from last tile in the chained solve's
 // order) for d = 1 .. depth (<= 3): depth * ceil(n/64) * 64 * 64 floats, M_d at

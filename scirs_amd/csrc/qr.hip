@@ -805,7 +805,8 @@ extern "C" int scirs_gpu_dlstsq(int rows, int cols, const double *a, int64_t lda
     SCIRS_HIP_CHECK(hipGetLastError());
     if ((rc = c.ensure_xtri(cols))) return finish(info, rc, t0);
     if ((rc = c.reset_flags(s))) return finish(info, rc, t0);
-    if ((rc = scirs_trsv_chain<double>(cols, 1, dR, pr, dy, 1, 0, 0, c.work, s))) return finish(info, rc, t0);
+    if ((rc = scirs_trsv_chain<double>(cols, 1, dR, pr, dy, 1, 0, 0, c.work, s, nullptr, nullptr, 1)))
+        return finish(info, rc, t0);
     int st = 0;
     if ((rc = c.read_flags(s, &st, nullptr))) return finish(info, rc, t0);
     resid_sq_kernel<<<(rows + 3) / 4, 256, 0, s>>>(dA, pa, rows, cols, db, dy, dsq);
