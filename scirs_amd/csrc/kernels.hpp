@@ -75,10 +75,12 @@ template <typename T> int scirs_sub_max_rows();
 // That sub-panel's interchanges, U12 = L11^-1 A12 and the update of columns
 // [ca, cb), its interchanges on columns [la, lb), and, ncomp > 0, the composition
 // of the ncomp lists at cpairs / cn (SCIRS_SUB_CTL counts apart) into one.
+// from_zero: each element's 32 products are summed from zero, else subtracted from it
+// one after the other.
 template <typename T>
-int scirs_sub_apply(T *A, long lda, int rows, int c0, int w, int ca, int cb, int la, int lb, const int *pairs,
-                    const int *npairs, int ncomp, const int *cpairs, const int *cn, int *out_pairs, int *out_n,
-                    ScirsWork &wk, hipStream_t s);
+int scirs_sub_apply(T *A, long lda, int rows, int c0, int w, int ca, int cb, int la, int lb, bool from_zero,
+                    const int *pairs, const int *npairs, int ncomp, const int *cpairs, const int *cn, int *out_pairs,
+                    int *out_n, ScirsWork &wk, hipStream_t s);
 
 enum { TSLU_MAXLEV = 6, TSLU_MAXNODE = 512, TSLU_MAP = 512 };
 

@@ -622,8 +622,11 @@ constexpr int ANT = 256, SC = 64, SP = SC + 2;   // threads, columns of a strip,
 // another workgroup may still read it.  Rank 32 per pass: latency-bound at small
 // sizes (12 to 20 us a launch for FP64 of up to 7000 rows), HBM-bound above.
 // A: the matrix; L11: the sub-panel's diagonal block (in columns that no workgroup writes).
-template <typename T>
-__global__ __launch_bounds__(ANT) void sub_apply_kernel(T *__restrict__ A, const T *__restrict__ L11, ApplyArgs<T> a)
+// ZERO: the products summed from zero, else subtracted from the element one by one (the
+// caller chooses; the sums' 16 registers more are kept out of the accumulation registers,
+// for three workgroups per CU either way: n = 1999 solve 4.08 ms, with two 4.15 ms).
+template <typename T, bool ZERO>
+__global__ __launch_bounds__(ANT, 3) void sub_apply_kernel(T *__restrict__ A, const T *__restrict__ L11, ApplyArgs<T> a)
 {
     if (*a.info != 0) return;
     typedef typename Mf<T>::V V4;
@@ -759,8 +762,8 @@ __global__ __launch_bounds__(ANT) void sub_apply_kernel(T *__restrict__ A, const
         }
         __syncthreads();
     }
-    // rank-32 update, the products subtracted one after the other in the order of the
-    // columns (lane group g, step i -> k = 4 i + g): every partial sum is then a Schur
+    // rank-32 update, the products in the order of the columns (lane group g, step i ->
+    // k = 4 i + g): subtracted one after the other, every partial sum is then a Schur
     // complement, which the pivoting keeps small.  In the order that lets a lane load its
     // eight L entries as one piece (k = 8 g + i) the factors of N(0,1) matrices of 64 to
     // 400 rows had 7 to 17 % more error.
@@ -796,6 +799,27 @@ __global__ __launch_bounds__(ANT) void sub_apply_kernel(T *__restrict__ A, const
             for (int i = 0; i < 8; ++i) lf[i] = 4 * i + grp < a.w ? -src[4 * i + grp] : (T)0;
         }
     };
+    // four tiles of one row block, two at a time where each needs a sum of its own
+    auto update = [&](const T (&lf)[8], V4 (&c4)[SC / 16]) {
+        if constexpr (ZERO) {
+#pragma unroll
+            for (int j = 0; j < SC / 16; j += 2) {
+                V4 sum[2] = {};
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) sum[h] = Mf<T>::mac(lf[i], uf[j + h][i], sum[h]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) c4[j + h] += sum[h];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < SC / 16; ++j)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) c4[j] = Mf<T>::mac(lf[i], uf[j][i], c4[j]);
+        }
+    };
     for (int rt = r0 + 16 * wave; rt < r1; rt += 64) {
         T lf[8];
         V4 acc[SC / 16];
@@ -807,10 +831,7 @@ __global__ __launch_bounds__(ANT) void sub_apply_kernel(T *__restrict__ A, const
                 const int r = min(rt + Mf<T>::row(grp, q), r1 - 1), cc = min(cs + 16 * j + l16, a.cb - 1);
                 acc[j][q] = A[(long)r * a.lda + cc];
             }
-#pragma unroll
-        for (int j = 0; j < SC / 16; ++j)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[j] = Mf<T>::mac(lf[i], uf[j][i], acc[j]);
+        update(lf, acc);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int r = rt + Mf<T>::row(grp, q);
@@ -835,10 +856,7 @@ __global__ __launch_bounds__(ANT) void sub_apply_kernel(T *__restrict__ A, const
                 const int e = min(16 * wave + Mf<T>::row(grp, q), nd - 1), cc = min(cs + 16 * j + l16, a.cb - 1);
                 acc[j][q] = A[(long)dsrc[e] * a.lda + cc];
             }
-#pragma unroll
-        for (int j = 0; j < SC / 16; ++j)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[j] = Mf<T>::mac(lf[i], uf[j][i], acc[j]);
+        update(lf, acc);
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -912,8 +930,8 @@ template int scirs_sub_panel<double>(double *, long, int, int, int, int *, int *
 template int scirs_sub_panel<float>(float *, long, int, int, int, int *, int *, int *, ScirsWork &, hipStream_t);
 
 template <typename T>
-int scirs_sub_apply(T *A, long lda, int rows, int c0, int w, int ca, int cb, int la, int lb, const int *pairs,
-                    const int *npairs, int ncomp, const int *cpairs, const int *cn, int *out_pairs, int *out_n,
+int scirs_sub_apply(T *A, long lda, int rows, int c0, int w, int ca, int cb, int la, int lb, bool from_zero,
+                    const int *pairs, const int *npairs, int ncomp, const int *cpairs, const int *cn, int *out_pairs, int *out_n,
                     ScirsWork &wk, hipStream_t s)
 {
     using namespace sub;
@@ -937,11 +955,13 @@ int scirs_sub_apply(T *A, long lda, int rows, int c0, int w, int ca, int cb, int
     a.label = wk.sub_label; a.info = wk.info;
     const int wgs = a.nstrip * a.nchunk + a.nleft + (ncomp > 0 ? 1 : 0);
     if (wgs == 0) return SCIRS_OK;
-    hipLaunchKernelGGL(sub_apply_kernel<T>, dim3(wgs), dim3(ANT), 0, s, A, (const T *)(A + (long)c0 * lda + c0), a);
+    const T *l11 = A + (long)c0 * lda + c0;
+    if (from_zero) hipLaunchKernelGGL((sub_apply_kernel<T, true>), dim3(wgs), dim3(ANT), 0, s, A, l11, a);
+    else hipLaunchKernelGGL((sub_apply_kernel<T, false>), dim3(wgs), dim3(ANT), 0, s, A, l11, a);
     SCIRS_HIP_CHECK(hipGetLastError());
     return SCIRS_OK;
 }
-template int scirs_sub_apply<double>(double *, long, int, int, int, int, int, int, int, const int *, const int *, int,
-                                     const int *, const int *, int *, int *, ScirsWork &, hipStream_t);
-template int scirs_sub_apply<float>(float *, long, int, int, int, int, int, int, int, const int *, const int *, int,
-                                    const int *, const int *, int *, int *, ScirsWork &, hipStream_t);
+template int scirs_sub_apply<double>(double *, long, int, int, int, int, int, int, int, bool, const int *, const int *,
+                                     int, const int *, const int *, int *, int *, ScirsWork &, hipStream_t);
+template int scirs_sub_apply<float>(float *, long, int, int, int, int, int, int, int, bool, const int *, const int *,
+                                    int, const int *, const int *, int *, int *, ScirsWork &, hipStream_t);
