@@ -4,6 +4,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "api_internal.hpp"
+#include "tags.hpp"
 #include "../../include/scirs_gpu.h"
 
 #include <chrono>
@@ -152,10 +153,10 @@ int Context::init(int dev)
                  tpu_b = 64 * 64 * sizeof(float), tpr_b = 64 * 64 * sizeof(float),
                  tpt_b = 64 * (size_t)kbmax * sizeof(float), tpv_b = 65 * sizeof(int),
                  tpm_b = (2 * (size_t)TSLU_MAP + 1) * sizeof(int);
-    const size_t sk_b = 2 * (size_t)SCIRS_SUB_AGENTS * 2 * 8, sr_b = 2 * (size_t)SCIRS_SUB_AGENTS * SCIRS_SUB_W * 2 * 8,
+    const size_t sx_b = (size_t)SCIRS_SUB_XCH_INTS * 4,
                  sc_b = (size_t)SCIRS_SUB_MAX * SCIRS_SUB_CTL * 4, sp_b = (size_t)SCIRS_SUB_MAX * SCIRS_SUB_PAIRS * 2 * 4,
                  sa_b = ((size_t)SCIRS_SUB_STRIPS + 1) * 4, sl_b = (size_t)SCIRS_SUB_ROWS * 4;
-    for (size_t b : {sk_b, sr_b, sc_b, sp_b, sa_b, sl_b}) bytes += (b + 255) & ~(size_t)255;
+    for (size_t b : {sx_b, sc_b, sp_b, sa_b, sl_b}) bytes += (b + 255) & ~(size_t)255;
     for (size_t b : {xw_b, xrow_b, xrj_b, flags_b, pairs_b, npairs_b, linv_b, tpc_b, tpn_b, tpu_b, tpr_b, tpt_b, tpt_b,
                      tpv_b, tpm_b})
         bytes += (b + 255) & ~(size_t)255;
@@ -186,8 +187,9 @@ int Context::init(int dev)
     work.tp_stage = (float *)take(tpt_b);
     work.tp_vlist = (int *)take(tpv_b);
     work.tp_map = (int *)take(tpm_b);
-    work.sub_key = (unsigned long long *)take(sk_b);
-    work.sub_row = (unsigned long long *)take(sr_b);
+    work.sub_key = (unsigned long long *)take(sx_b);
+    work.sub_row = work.sub_key + 2 * SCIRS_SUB_AGENTS * 2;
+    work.sub_next = 1;
     work.sub_ctl = (int *)take(sc_b);
     work.sub_pairs = (int *)take(sp_b);
     work.sub_arrive = (int *)take(sa_b);
@@ -785,9 +787,7 @@ static int clear_tags(ScirsWork &w, hipStream_t s)
 {
     struct Buf { unsigned long long *p; size_t words; };
     const Buf bufs[] = {{w.xw, w.xw_words}, {w.xrow, w.xrow_words}, {w.xrj, w.xrj_words}, {w.xtri, w.xtri_words},
-                        {w.tp_cand, (size_t)TSLU_MAXLEV * TSLU_MAXNODE * 65},
-                        {w.sub_key, (size_t)2 * SCIRS_SUB_AGENTS * 2},
-                        {w.sub_row, (size_t)2 * SCIRS_SUB_AGENTS * SCIRS_SUB_W * 2}};
+                        {w.tp_cand, (size_t)TSLU_MAXLEV * TSLU_MAXNODE * 65}};
     for (const Buf &b : bufs) {
         if (!b.p || !b.words) continue;
         for (size_t off = 0; off < 2 * b.words; off += (size_t)1 << 30) {
@@ -814,12 +814,8 @@ extern "C" int scirs_gpu_seq_plan(unsigned next, unsigned span, unsigned *base, 
     // a launch tags its words with base .. base + span - 1 (never 0, the value of
     // a cleared word); when that range would reach the top of the 32-bit count,
     // the caller clears the tagged buffers and the count restarts at 1
-    int reset = 0;
-    if (next == 0u || span == 0u || next > 0xFFFFFFFFu - span) {
-        next = 1u;
-        reset = 1;
-    }
-    *base = next;
-    *next_out = next + (span ? span : 1u);
-    return reset;
+    const tags::Range r = tags::draw(next, span, 0xFFFFFFFFu);
+    *base = r.base;
+    *next_out = r.next;
+    return r.clear ? 1 : 0;
 }

@@ -50,8 +50,9 @@ struct ScirsWork {
     int *tp_vlist;             // [64 + 1] positions the displaced rows move to, then their count
     int *tp_map;               // [2 * TSLU_MAP] (position, original row) of the panel's moved rows, then a count
     // sub-panel factorisation (subpanel.hip)
-    unsigned long long *sub_key;   // [2][SCIRS_SUB_AGENTS][2] candidates (sequence-tagged words)
+    unsigned long long *sub_key;   // [2][SCIRS_SUB_AGENTS][2] candidates (tagged words); sub_row follows them
     unsigned long long *sub_row;   // [2][SCIRS_SUB_AGENTS][SCIRS_SUB_W][2] their rows
+    unsigned sub_next;             // next tag of these two
     int *sub_ctl;                  // [SCIRS_SUB_MAX][SCIRS_SUB_CTL] election of the die, count of moved rows
     int *sub_pairs;                // [SCIRS_SUB_MAX][SCIRS_SUB_PAIRS][2] moved rows of a sub-panel
     int *sub_arrive;               // [SCIRS_SUB_STRIPS] arrival counts (zero between launches)
@@ -61,9 +62,11 @@ struct ScirsWork {
 
 // Sub-panel width, waves of its exchange, moved rows at most, sub-panels per
 // factorisation, control words of one (8 dies' counts 32 apart, the elected die,
-// the moved-row count), strips of a sub-panel update, rows of the matrix.
+// the moved-row count), strips of a sub-panel update, rows of the matrix, 32-bit words
+// of the exchange (candidates and rows).
 enum { SCIRS_SUB_W = 32, SCIRS_SUB_AGENTS = 128, SCIRS_SUB_PAIRS = 64, SCIRS_SUB_MAX = 2048, SCIRS_SUB_CTL = 320,
-       SCIRS_SUB_COUNT = 288, SCIRS_SUB_STRIPS = 2048, SCIRS_SUB_ROWS = 1 << 16 };
+       SCIRS_SUB_COUNT = 288, SCIRS_SUB_STRIPS = 2048, SCIRS_SUB_ROWS = 1 << 16,
+       SCIRS_SUB_XCH_INTS = 2 * 2 * SCIRS_SUB_AGENTS * 2 * (1 + SCIRS_SUB_W) };
 
 // Factor columns c0 .. c0 + w - 1 (w <= 32), rows c0 .. rows - 1, with partial
 // pivoting; the rows that move (destination, source) go to pairs, their number is

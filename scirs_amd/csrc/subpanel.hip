@@ -36,6 +36,7 @@
 #include "kernels.hpp"
 #include "lanes.hpp"
 #include "prof.hpp"
+#include "tags.hpp"
 
 #include "api_internal.hpp"
 
@@ -165,7 +166,7 @@ template <typename T> struct PanelArgs {
     int G;               // waves that hold rows
     u64 *key, *row;      // [2][GMAX][2] candidates, [2][GMAX][32][2] their rows (tagged words)
     int *elect;          // per-die registration counts (128 bytes apart), then the elected die + 1; zeroed
-    u32 seq;
+    u32 seq;             // tag of column 0
     int *pairs, *npairs; // the moved rows (destination, source), absolute; *npairs zeroed
     int *info; double *info_val; int *abort;
     u32 spin_limit;
@@ -232,8 +233,7 @@ template <typename T, int R, int J> __device__ __forceinline__ void row_out(cons
 
 // Column J.  NW > 0: one workgroup of at most NW waves, exchange through LDS.
 // NW = 0: wave g of A.G, exchange through the die's L2 in 64-bit words that carry the
-// column's 32-bit tag beside 32 bits of data (the candidate's second word: 16 tag
-// bits and the position), NS candidates per lane.  Bounded polls: a wave that gives
+// column's tag (tags.hpp), NS candidates per lane.  Bounded polls: a wave that gives
 // up stops the panel.  A wave's update of the columns beyond the current block waits
 // until its candidate is on its way, so that it runs in the exchange's shadow.
 template <typename T, int R, int NS, int NW, int J>
@@ -279,8 +279,8 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
 #pragma unroll
         for (int x = 0; x < R; ++x)
             if (win[x]) {
-                put(ks, ((u64)tag << 32) | gm);
-                put(ks + 1, ((u64)((tag << 16) | ((u32)S.pos[x] & 0xffffu)) << 32) | V::lo(S.a[x][J]));
+                put(ks, tags::value_word(tag, gm));
+                put(ks + 1, tags::position_word(tag, (u32)S.pos[x], V::lo(S.a[x][J])));
             }
 #pragma unroll
         for (int x = 0; x < R; ++x) {
@@ -319,17 +319,16 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
         while (true) {
             bool ok = true;
 #pragma unroll
-            for (int s = 0; s < NS; ++s)
-                ok = ok && (u32)(k0[s] >> 32) == tag && (u32)(k1[s] >> 48) == (tag & 0xffffu);
+            for (int s = 0; s < NS; ++s) ok = ok && tags::current(k0[s], k1[s], tag);
             if (__builtin_expect(bal(ok) == ~0ull, 1)) break;
             if (give_up()) { late = true; break; }
             poll();
         }
-        u32 kh = (u32)k0[0], kl = (u32)k1[0], kp = (u32)(k1[0] >> 32) & 0xffffu;
+        u32 kh = (u32)k0[0], kl = (u32)k1[0], kp = tags::position(k1[0]);
         int slot = 0;
 #pragma unroll
         for (int s = 1; s < NS; ++s) {
-            const u32 h2 = (u32)k0[s], l2 = (u32)k1[s], p2 = (u32)(k1[s] >> 32) & 0xffffu;
+            const u32 h2 = (u32)k0[s], l2 = (u32)k1[s], p2 = tags::position(k1[s]);
             const bool bt = h2 > kh || (h2 == kh && (l2 > kl || (l2 == kl && p2 < kp)));
             kh = bt ? h2 : kh;
             kl = bt ? l2 : kl;
@@ -902,7 +901,7 @@ int scirs_sub_panel(T *A, long lda, int rows, int c0, int w, int *pairs, int *np
     PanelArgs<T> pa;
     pa.A = A + (long)c0 * lda + c0; pa.lda = lda; pa.top = c0; pa.m = rows - c0; pa.w = w;
     pa.key = wk.sub_key; pa.row = wk.sub_row; pa.elect = elect;
-    if (int rc = scirs_next_seq(wk, W, s, &pa.seq)) return rc;
+    pa.seq = 0;
     pa.pairs = pairs; pa.npairs = npairs;
     pa.info = wk.info; pa.info_val = wk.info_val; pa.abort = wk.abort; pa.spin_limit = wk.spin_limit;
     auto waves = [&](int r) { return (pa.m + 64 * r - 1) / (64 * r); };
@@ -913,6 +912,12 @@ int scirs_sub_panel(T *A, long lda, int rows, int c0, int w, int *pairs, int *np
     if constexpr (!f64) {
         if (waves(2) <= 8) { pa.G = waves(2); return launch_panel<T, 2, 1, 8>(pa, s); }
     }
+    // from here on the waves exchange through the die's L2, by tags
+    const tags::Range r = tags::draw(wk.sub_next, W, tags::CANDIDATE_TOP);
+    if (r.clear)
+        if (int rc = scirs_fill_int((int *)wk.sub_key, SCIRS_SUB_XCH_INTS, 0, s)) return rc;
+    wk.sub_next = r.next;
+    pa.seq = r.base;
     if (pa.G <= 64) return launch_panel<T, 1, 1, 0>(pa, s);
     pa.G = waves(2);
     if (pa.G <= 64) return launch_panel<T, 2, 1, 0>(pa, s);
