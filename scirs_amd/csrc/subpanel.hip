@@ -33,6 +33,7 @@
 // one row per thread, LDS broadcasts and a rolled loop), 2000 rows 41 us and 8192
 // rows 50 us (160 us with one exchange per column over the whole device).
 #include "common.hpp"
+#include "elect.hpp"
 #include "kernels.hpp"
 #include "lanes.hpp"
 #include "prof.hpp"
@@ -455,11 +456,41 @@ __device__ __forceinline__ void steps(Rows<T, R> &S, const PanelArgs<T> &A, int 
     }
 }
 
+// elect::place on the device: eight counts 128 bytes apart, then the elected die + 1
+struct Ballot {
+    int *count;
+    int *info, *abort;
+    int top, die;   // die: HW_REG_XCC_ID, bits 0..3
+    __device__ bool stopped() const
+    {
+        return __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    }
+    __device__ int add()
+    {
+        return __hip_atomic_fetch_add(count + 32 * die, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ void claim()
+    {
+        int none = 0;
+        __hip_atomic_compare_exchange_strong(count + 32 * 8, &none, die + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ int winner() const
+    {
+        return __hip_atomic_load(count + 32 * 8, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ int mine() const { return die + 1; }
+    __device__ void timed_out()
+    {
+        __hip_atomic_store(abort, top + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+};
+
 // NW = 0: workgroups of 256 threads, each wave an agent of the exchange
 template <typename T, int R, int NS, int NW>
 __global__ __launch_bounds__(NW ? 64 * NW : 256, 2) void sub_panel_kernel(PanelArgs<T> A)
 {
-    if (*A.info != 0) return;
     constexpr int NWV = NW ? NW : 4;
     constexpr int E = 16 / (int)sizeof(T), NE = 128 / (int)sizeof(T), PE = NE + E;   // 128-byte row segments
     typedef typename Vec16<T>::type V;
@@ -473,29 +504,16 @@ __global__ __launch_bounds__(NW ? 64 * NW : 256, 2) void sub_panel_kernel(PanelA
     int g = wave;
     if constexpr (NW == 0) {
         if (t == 0) {
-            const int gw = (A.G + 3) / 4;   // places
-            const int x = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7;   // HW_REG_XCC_ID, bits 0..3
-            const int tk = __hip_atomic_fetch_add(A.elect + 32 * x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            int *won = A.elect + 32 * 8;
-            if (tk == gw - 1) {
-                int none = 0;
-                __hip_atomic_compare_exchange_strong(won, &none, x + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
-            }
-            int wn = 0;
-            for (u32 q = 0; q < A.spin_limit && wn == 0; ++q)
-                wn = __hip_atomic_load(won, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (wn == 0) {
-                __hip_atomic_store(A.abort, A.top + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(A.info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            s_g = (wn == x + 1 && tk < gw) ? tk : -1;
+            Ballot m{A.elect, A.info, A.abort, A.top, (int)(__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 7)};
+            s_g = elect::place(m, (A.G + 3) / 4, A.spin_limit);
         }
         __syncthreads();
         if (s_g < 0) return;
         g = 4 * s_g + wave;
         if (g >= A.G) return;   // (no barrier follows: the waves are independent from here on)
     } else {
+        // (one workgroup: nobody else sets info while it runs)
+        if (*A.info != 0) return;
         if (t < 32) L.key[t >> 4][t & 15] = uint4{0, 0, 0, 0};
         __syncthreads();
     }
