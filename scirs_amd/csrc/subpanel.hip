@@ -79,8 +79,6 @@ template <int N> __device__ __forceinline__ u32 group_max(u32 v)
 __device__ __forceinline__ u32 rl(u32 v, int k) { return (u32)__builtin_amdgcn_readlane((int)v, k); }
 __device__ __forceinline__ u64 bal(bool c) { return __builtin_amdgcn_ballot_w64(c); }
 
-// The search key of a value is its top word without the sign: |v| ordered, except
-// that FP64 values equal in their top 20 mantissa bits need the lower word too.
 // a's lanes with bit N set <-> b's lanes with bit N clear
 template <int N, typename T> __device__ __forceinline__ void swap_groups(T &a, T &b)
 {
@@ -108,6 +106,10 @@ template <int N, typename T> __device__ __forceinline__ void swap_groups(T &a, T
     }
 }
 
+// The search key of a value is its top word without the sign, |v| ordered, except that
+// FP64 values equal in their top 20 mantissa bits need the lower word too; minus (the word
+// of infinity + 1), which wraps every number above the NaN: these compare with nothing
+// (lapack.rs:95-104), so they are candidates only where nothing else is left.
 template <typename T> struct Val;
 template <> struct Val<double> {
     static __device__ __forceinline__ u32 hi(double v) { return (u32)((u64)__double_as_longlong(v) >> 32); }
@@ -151,6 +153,9 @@ template <> struct Val<float> {
     static constexpr u32 big_hi = 0x7c000000u;
 };
 
+template <typename T> __host__ __device__ constexpr u32 to_key(u32 hi) { return hi - Val<T>::inf_hi - 1u; }
+template <typename T> __host__ __device__ constexpr u32 from_key(u32 key) { return key + Val<T>::inf_hi + 1u; }
+
 __device__ __forceinline__ void put(u64 *p, u64 v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -179,10 +184,11 @@ template <typename T, int R> struct Rows {
     u32 live[R];     // 31 while the row can still be picked, 0 after (the width of the key's bit field)
     T l[R];          // multipliers of the last column
     T pr[W / 16];    // its pivot row: lane l holds elements l % 16 and 16 + l % 16
+    T odd;           // zero until a pivot row holds an infinity or a NaN
     bool stop;
 };
-template <typename T, int NW> struct Xch {
-    alignas(16) T row[2][NW][W];
+template <typename T> struct Xch {
+    alignas(16) T row[W][W];   // the pivot rows (many workgroups: each wave writes them all, the same)
     uint4 key[2][16];
 };
 
@@ -238,7 +244,7 @@ template <typename T, int R, int J> __device__ __forceinline__ void row_out(cons
 // up stops the panel.  A wave's update of the columns beyond the current block waits
 // until its candidate is on its way, so that it runs in the exchange's shadow.
 template <typename T, int R, int NS, int NW, int J>
-__device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g, T *lr, Xch<T, NW ? NW : 1> *L)
+__device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g, T *lr, Xch<T> *L)
 {
     typedef Val<T> V;
     const int lane = threadIdx.x & 63;
@@ -247,7 +253,7 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
     bool win[R];
 #pragma unroll
     for (int x = 0; x < R; ++x) {
-        h[x] = __builtin_amdgcn_ubfe(V::hi(S.a[x][J]), 0, S.live[x]);
+        h[x] = to_key<T>(__builtin_amdgcn_ubfe(V::hi(S.a[x][J]), 0, S.live[x]));
         hm = max(hm, h[x]);
     }
     const u32 gm = wave_max_u32(hm);
@@ -265,7 +271,7 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
             win[x] = win[x] && S.live[x] != 0;
         }
         tie_break<R>(win, lo, S.pos);
-        if (gm == 0) {   // a zero column, or no row left: still one candidate
+        if (gm <= to_key<T>(0)) {   // zeros and NaN, or no row left: still one candidate
             bool any = false;
 #pragma unroll
             for (int x = 0; x < R; ++x) any = any || win[x];
@@ -366,7 +372,9 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
             if (__builtin_expect(bal(ok) == ~0ull, 1)) break;
             if (late || give_up()) { late = true; break; }
         }
-        if (__builtin_expect(S.stop || late || khi - V::eps_hi > V::inf_hi - V::eps_hi, 0)) {
+#pragma unroll
+        for (int k = J / 16; k < W / 16; ++k) L->row[J][16 * k + (lane & 15)] = S.pr[k];
+        if (__builtin_expect(S.stop || late || khi < to_key<T>(V::eps_hi), 0)) {
             if (!S.stop && lane == 0) {
                 if (late) {
                     // the 1-based column whose exchange timed out; info != 0 stops what is queued
@@ -374,7 +382,7 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
                     __hip_atomic_store(A.info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 } else if (g == 0) {
                     *A.info = A.top + J + 1;
-                    *A.info_val = (double)V::make(khi, rl(kl, wl));
+                    *A.info_val = khi > to_key<T>(0) ? (double)V::make(from_key<T>(khi), rl(kl, wl)) : 0.0;
                 }
             }
             S.stop = true;
@@ -406,20 +414,20 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
         if (wl == wave) {
 #pragma unroll
             for (int x = 0; x < R; ++x)
-                if (win[x]) row_out<T, R, J>(S, x, L->row[b][0]);
+                if (win[x]) row_out<T, R, J>(S, x, L->row[J]);
         }
         khi = rl(k.x, wl);
         p = (int)rl(k.z, wl);
-        if (__builtin_expect(S.stop || khi - V::eps_hi > V::inf_hi - V::eps_hi, 0)) {
+        if (__builtin_expect(S.stop || khi < to_key<T>(V::eps_hi), 0)) {
             if (!S.stop && threadIdx.x == 0) {
                 *A.info = A.top + J + 1;
-                *A.info_val = (double)V::make(khi, rl(k.y, wl));
+                *A.info_val = khi > to_key<T>(0) ? (double)V::make(from_key<T>(khi), rl(k.y, wl)) : 0.0;
             }
             S.stop = true;
         }
         __syncthreads();
 #pragma unroll
-        for (int q = J / 16; q < W / 16; ++q) S.pr[q] = L->row[b][0][16 * q + (lane & 15)];
+        for (int q = J / 16; q < W / 16; ++q) S.pr[q] = L->row[J][16 * q + (lane & 15)];
     }
     if (__builtin_expect(S.stop, 0)) {
 #pragma unroll
@@ -436,7 +444,7 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
             S.pos[x] = hit ? J : (ps == J ? p : ps);   // the interchange of positions J and p
             S.live[x] = hit ? 0u : S.live[x];
             T q = V::div(S.a[x][J], piv, r);
-            if (__builtin_expect(khi >= V::big_hi, 0)) q = S.a[x][J] / piv;
+            if (__builtin_expect(khi >= to_key<T>(V::big_hi), 0)) q = S.a[x][J] / piv;
             S.a[x][J] = S.live[x] ? q : S.a[x][J];
             S.l[x] = S.live[x] ? q : (T)0;
         }
@@ -446,9 +454,11 @@ __device__ __forceinline__ void step(Rows<T, R> &S, const PanelArgs<T> &A, int g
 #pragma unroll
         for (int x = 0; x < R; ++x) fmac_row<(J + 1) & 15, 1>(&S.a[x][J + 1], S.pr[(J + 1) >> 4], S.l[x]);
     }
+#pragma unroll
+    for (int q = J / 16; q < W / 16; ++q) S.odd = fma((T)0, S.pr[q], S.odd);
 }
 template <typename T, int R, int NS, int NW, int J>
-__device__ __forceinline__ void steps(Rows<T, R> &S, const PanelArgs<T> &A, int g, T *lr, Xch<T, NW ? NW : 1> *L)
+__device__ __forceinline__ void steps(Rows<T, R> &S, const PanelArgs<T> &A, int g, T *lr, Xch<T> *L)
 {
     if constexpr (J < W) {
         if (J < A.w) step<T, R, NS, NW, J>(S, A, g, lr, L);
@@ -498,7 +508,7 @@ __global__ __launch_bounds__(NW ? 64 * NW : 256, 2) void sub_panel_kernel(PanelA
     __shared__ __align__(16) T seg[NWV][32 * PE];   // 32 rows of one segment, per wave
     __shared__ __align__(16) T lrow[NWV][W];
     __shared__ int dpos[NWV][32];
-    __shared__ Xch<T, NW ? NW : 1> L;
+    __shared__ Xch<T> L;
     __shared__ int s_g;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     int g = wave;
@@ -566,6 +576,7 @@ __global__ __launch_bounds__(NW ? 64 * NW : 256, 2) void sub_panel_kernel(PanelA
         }
     }
     S.stop = false;
+    S.odd = (T)0;
     steps<T, R, NS, NW, 0>(S, A, g, lrow[wave], &L);
     // rows out, to their final positions, the same way (every row was read before the
     // first exchange of the panel ended)
@@ -603,6 +614,17 @@ __global__ __launch_bounds__(NW ? 64 * NW : 256, 2) void sub_panel_kernel(PanelA
                     }
                 }
             }
+    // A finished row takes part in the later updates with multiplier zero, which changes it
+    // if the pivot row of such an update is infinite or NaN: its later columns are those
+    // that it had as the pivot row.
+    if (__builtin_expect(bal(S.odd != (T)0) != 0, 0)) {
+        __builtin_amdgcn_s_waitcnt(0);   // behind the rows as they went out
+#pragma unroll
+        for (int x = 0; x < R; ++x)
+            if (S.live[x] == 0 && S.pos[x] >= 0)
+#pragma unroll 1
+                for (int d = S.pos[x], c = d + 1; c < A.w; ++c) A.A[(long)d * A.lda + c] = L.row[d][c];
+    }
 #pragma unroll
     for (int x = 0; x < R; ++x) {
         const int row = base + 64 * x + lane;
