@@ -136,12 +136,15 @@ template <typename T, int J> __device__ __forceinline__ bool chol_column(T (&a)[
     }
     return true;
 }
-// columns J .. 31; the failing column, or -1
-template <typename T, int J> __device__ __forceinline__ int chol_columns(T (&a)[CP_B], T &dv)
+// columns J .. 31 of a step with `cols` columns left (looked at every eighth: the others
+// are the identity's); the failing column, or -1
+template <typename T, int J> __device__ __forceinline__ int chol_columns(T (&a)[CP_B], T &dv, int cols)
 {
     if constexpr (J < CP_B) {
+        if constexpr (J > 0 && J % 8 == 0)
+            if (J >= cols) return -1;
         if (!chol_column<T, J>(a, dv)) return J;
-        return chol_columns<T, J + 1>(a, dv);
+        return chol_columns<T, J + 1>(a, dv, cols);
     } else {
         return -1;
     }
@@ -224,7 +227,7 @@ template <typename T> __global__ __launch_bounds__(NT, 2) void chol_panel_kernel
         const bool active = wave == 3 || wave >= jb;   // the wave's group lies below the diagonal rows
         if (active) {
             T dv;
-            const int f = chol_columns<T, 0>(a, dv);
+            const int f = chol_columns<T, 0>(a, dv, g.kb - B * jb);
             if (f >= 0) {
                 if (lane == 0) s_fail = 1;
                 if (wave == 3 && lane == 0 && blockIdx.x == 0) {
