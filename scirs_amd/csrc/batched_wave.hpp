@@ -222,6 +222,17 @@ __device__ __forceinline__ void load16(const float *row, float *v)
     }
 }
 
+// v[e], k = 4 grp + e, to k = 4 e + grp
+__device__ __forceinline__ void column_order(f4 &v)
+{
+    float w[4] = {v[0], v[1], v[2], v[3]};
+    lanes::swap_groups<32>(w[0], w[2]);
+    lanes::swap_groups<32>(w[1], w[3]);
+    lanes::swap_groups<16>(w[0], w[1]);
+    lanes::swap_groups<16>(w[2], w[3]);
+    v = f4{w[0], w[1], w[2], w[3]};
+}
+
 // The update of columns [k0 + KK, cend) behind KK = 16 or 32 finished columns, 64 of them
 // at a time; LU first solves U12 = L11^-1 A12 (lane = column).
 template <bool CHOL, int KK>
@@ -239,7 +250,7 @@ __device__ __forceinline__ void update(int np, int k0, int cend, float *W, const
     }
     for (int c0 = k1; c0 < cend; c0 += 64) {
         const int nct = min(4, (cend - c0) / KB);
-        float ua[4][KK / 4];      // block ct: element (k = 16 (i / 4) + 4 grp + i % 4, column l16) of U12, or of L21^T
+        float ua[4][KK / 4];      // block ct: element (k, column l16) of U12, k = 4 i + grp, or of L21^T, k = 16 (i / 4) + 4 grp + i % 4
         if constexpr (CHOL) {
 #pragma unroll
             for (int ct = 0; ct < 4; ++ct)
@@ -275,7 +286,7 @@ __device__ __forceinline__ void update(int np, int k0, int cend, float *W, const
             for (int ct = 0; ct < 4; ++ct)
 #pragma unroll
                 for (int i = 0; i < KK / 4; ++i)
-                    ua[ct][i] = ush[(KB * (i / 4) + 4 * grp + i % 4) * LU_ROW + ct * KB + l16];
+                    ua[ct][i] = ush[(4 * i + grp) * LU_ROW + ct * KB + l16];
             wsync();
         }
         // RB row blocks at a time, all their loads ahead of the products
@@ -290,6 +301,14 @@ __device__ __forceinline__ void update(int np, int k0, int cend, float *W, const
 #pragma unroll
                 for (int g = 0; g < KK / KB; ++g)
                     lv[h][g] = *reinterpret_cast<const f4 *>(row[h] + k0 + g * KB + 4 * grp);
+            }
+            // LU: the products in the order of the columns, whose partial sums the pivoting
+            // keeps small.  Lane group and register exchange their two bits of k.
+            if (!CHOL) {
+#pragma unroll
+                for (int h = 0; h < RB; ++h)
+#pragma unroll
+                    for (int g = 0; g < KK / KB; ++g) column_order(lv[h][g]);
             }
 #pragma unroll
             for (int h = 0; h < RB; ++h)
@@ -592,20 +611,30 @@ __device__ __forceinline__ Result refine(int n, int np, int nrhs, int j0, int nr
         rn = 0.0;
         nan = false;
         for (int r0 = 0; r0 < n; r0 += 2 * KB) {
-            // two row blocks; two partial sums per element: shorter chains, and less
-            // rounding in the residual
+            // two row blocks; each 32 columns in eight sums of four products (Cholesky: four of
+            // eight), added up in pairs.  A matrix-core step rounds after each of its products, so two
+            // sums along the whole row round n times at their full size (mean error of general systems of 8 to
+            // 256 rows, kappa = 1e3: 2.1e-14 so, 1.2e-14 as it is).
             const double *row[2] = {A + (long)min(r0 + l16, n - 1) * n, A + (long)min(r0 + KB + l16, n - 1) * n};
-            d4 part[2][2] = {};
+            d4 total[2] = {};
 #pragma unroll 2
             for (int kc = 0; kc < n; kc += 32) {
-                double v[2][8];
+                double v[2][8], xv[8];
                 load8(row[0], kc, grp, n, v[0]);
                 load8(row[1], kc, grp, n, v[1]);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const double xv = col ? xc[kc + 8 * (i / 2) + 2 * grp + i % 2] : 0.0;
+                for (int i = 0; i < 8; ++i) xv[i] = col ? xc[kc + 8 * (i / 2) + 2 * grp + i % 2] : 0.0;
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) part[h][i & 1] = lanes::Mf<double>::mac(v[h][i], xv, part[h][i & 1]);
+                for (int h = 0; h < 2; ++h) {
+                    constexpr int NS = CHOL ? 4 : 8;   // (eight cost the Cholesky kernel its third wave per SIMD)
+                    d4 part[NS] = {};
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) part[i % NS] = lanes::Mf<double>::mac(v[h][i], xv[i], part[i % NS]);
+#pragma unroll
+                    for (int s = 1; s < NS; s *= 2)
+#pragma unroll
+                        for (int i = 0; i < NS; i += 2 * s) part[i] += part[i + s];
+                    total[h] += part[0];
                 }
             }
 #pragma unroll
@@ -614,7 +643,7 @@ __device__ __forceinline__ Result refine(int n, int np, int nrhs, int j0, int nr
                 for (int q = 0; q < 4; ++q) {
                     const int r = r0 + h * KB + grp + 4 * q;
                     if (r < n && col) {
-                        const double rv = Bc[(long)r * nrhs] - (part[h][0][q] + part[h][1][q]);
+                        const double rv = Bc[(long)r * nrhs] - total[h][q];
                         rn = fmax(rn, fabs(rv));
                         nan |= rv != rv;
                         dc[CHOL ? r : imap[r]] = rv;

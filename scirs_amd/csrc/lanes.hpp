@@ -45,6 +45,33 @@ template <int I0, int K, typename T> __device__ __forceinline__ void fmac_row(T 
     }
 }
 
+// a's lanes with bit N set <-> b's lanes with bit N clear
+template <int N, typename T> __device__ __forceinline__ void swap_groups(T &a, T &b)
+{
+    auto word = [](unsigned &x, unsigned &y) {
+        if constexpr (N == 32) {
+            const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+            x = r[0]; y = r[1];
+        } else {
+            const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+            x = r[0]; y = r[1];
+        }
+    };
+    if constexpr (sizeof(T) == 8) {
+        const unsigned long long p = (unsigned long long)__double_as_longlong(a), q = (unsigned long long)__double_as_longlong(b);
+        unsigned pl = (unsigned)p, ph = (unsigned)(p >> 32), ql = (unsigned)q, qh = (unsigned)(q >> 32);
+        word(pl, ql);
+        word(ph, qh);
+        a = __longlong_as_double((long long)(((unsigned long long)ph << 32) | pl));
+        b = __longlong_as_double((long long)(((unsigned long long)qh << 32) | ql));
+    } else {
+        unsigned p = __float_as_uint(a), q = __float_as_uint(b);
+        word(p, q);
+        a = __uint_as_float(p);
+        b = __uint_as_float(q);
+    }
+}
+
 template <typename T> struct Vec16;
 template <> struct Vec16<double> { typedef double type __attribute__((ext_vector_type(2))); };
 template <> struct Vec16<float> { typedef float type __attribute__((ext_vector_type(4))); };

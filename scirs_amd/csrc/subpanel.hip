@@ -79,33 +79,6 @@ template <int N> __device__ __forceinline__ u32 group_max(u32 v)
 __device__ __forceinline__ u32 rl(u32 v, int k) { return (u32)__builtin_amdgcn_readlane((int)v, k); }
 __device__ __forceinline__ u64 bal(bool c) { return __builtin_amdgcn_ballot_w64(c); }
 
-// a's lanes with bit N set <-> b's lanes with bit N clear
-template <int N, typename T> __device__ __forceinline__ void swap_groups(T &a, T &b)
-{
-    auto word = [](u32 &x, u32 &y) {
-        if constexpr (N == 32) {
-            const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-            x = r[0]; y = r[1];
-        } else {
-            const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
-            x = r[0]; y = r[1];
-        }
-    };
-    if constexpr (sizeof(T) == 8) {
-        const u64 p = (u64)__double_as_longlong(a), q = (u64)__double_as_longlong(b);
-        u32 pl = (u32)p, ph = (u32)(p >> 32), ql = (u32)q, qh = (u32)(q >> 32);
-        word(pl, ql);
-        word(ph, qh);
-        a = __longlong_as_double((long long)(((u64)ph << 32) | pl));
-        b = __longlong_as_double((long long)(((u64)qh << 32) | ql));
-    } else {
-        u32 p = __float_as_uint(a), q = __float_as_uint(b);
-        word(p, q);
-        a = __uint_as_float(p);
-        b = __uint_as_float(q);
-    }
-}
-
 // The search key of a value is its top word without the sign, |v| ordered, except that
 // FP64 values equal in their top 20 mantissa bits need the lower word too; minus (the word
 // of infinity + 1), which wraps every number above the NaN: these compare with nothing
