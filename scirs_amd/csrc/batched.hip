@@ -1,5 +1,5 @@
 // Batched solves of many independent small systems of uneven size
-// (n <= 256) in one launch.
+// (n <= 256) in one call.
 //
 // There is no batched solve in the reference (scirs2-linalg/src/batch/mod.rs
 // offers matmul/matvec/add/sum only); each system follows the reference's
@@ -20,7 +20,8 @@
 // every system through FP32 and the refinement, one wave each
 // (batched_wave.hpp); it marks those that need FP64, and a second launch takes
 // these from a queue: n > wave_max by a 256-thread workgroup, smaller ones one
-// per wave.  Without any it ends at once.
+// per wave.  Without any it ends at once.  Batches whose workspace passes
+// BATCH_WORK_MB take these launches chunk by chunk.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "prof.hpp"
@@ -363,6 +364,10 @@ __global__ void batched_reset_kernel(unsigned *counter) { counter[threadIdx.x] =
 // (NMAX / 4 is what a wave's slice of LDS holds; 4000 systems of 33 to 64 rows: 1.4 ms, by
 // workgroups 3.1; 8000 of 8 to 32: 0.86 and 1.9)
 constexpr int FP64_WAVE_MAX = NMAX / 4;
+// Workspace of a batch, MiB: a padded system takes up to 40 times what its matrix does
+// (5 KB for n <= 16), so larger batches run in several chunks that share it.  Half of
+// the factors of 65,000 systems of 256 rows; a chunk of systems of 16 rows is 1.6 million.
+constexpr long BATCH_WORK_MB = 8192;
 constexpr int NEED_FP64 = -1000;     // status between the two launches
 
 // systems order[0..gridDim.x), all of one kind
@@ -439,12 +444,16 @@ __global__ __launch_bounds__(NT) void batched_solve_kernel(BatchArgs a)
 
 namespace {
 
+// Systems that share the workspace: order[first .. first + count), of which `general` are
+// general ones (kinds: those first, then the positive definite ones, each by size).
+struct BatchChunk { int first, count, general; };
+
 struct BatchPlan {
     uint64_t key = 0;
     int batch = 0;
     BatchDesc *d_desc = nullptr;
-    int *d_order = nullptr, *d_kinds = nullptr;   // by size; general systems by size, then SPD ones by size
-    int general = 0;
+    int *d_order = nullptr, *d_kinds = nullptr;   // by size; within a chunk by kind and size
+    std::vector<BatchChunk> chunks;
     long *d_offP = nullptr;
     int *d_status = nullptr, *d_iters = nullptr;
     double *d_bwd = nullptr;
@@ -495,20 +504,25 @@ int launch_batch(BatchPlan &pl, const double *dA, const double *dB, double *dX, 
                  double tol_scale, hipStream_t s)
 {
     BatchArgs a;
-    a.desc = pl.d_desc; a.order = pl.d_order; a.batch = pl.batch;
+    a.desc = pl.d_desc;
     a.A = dA; a.B = dB; a.X = dX; a.work = pl.d_work; a.perm = pl.d_perm; a.offP = pl.d_offP;
     a.status = pl.d_status; a.iters = pl.d_iters; a.bwd = pl.d_bwd; a.counter = pl.d_counter;
     a.wave_max = wave_max; a.max_iter = max_iter; a.tol_scale = tol_scale;
-    hipLaunchKernelGGL(batched_reset_kernel, dim3(1), dim3(2), 0, s, pl.d_counter);
-    if (pl.general)
-        hipLaunchKernelGGL(batched_wave_kernel<false>, dim3(pl.general), dim3(64), wave::lds_bytes(pl.nmax), s, a,
-                           pl.d_kinds);
-    if (pl.general < pl.batch)
-        hipLaunchKernelGGL(batched_wave_kernel<true>, dim3(pl.batch - pl.general), dim3(64), wave::lds_bytes(pl.nmax),
-                           s, a, pl.d_kinds + pl.general);
-    // a persistent grid: one workgroup per CU (LDS allows one) pulls work from the queue
-    const int grid = std::min(pl.batch, scirs::ctx().cu_count);
-    hipLaunchKernelGGL(batched_solve_kernel, dim3(grid), dim3(NT), 0, s, a);
+    for (const BatchChunk &ch : pl.chunks) {
+        a.order = pl.d_order + ch.first;
+        a.batch = ch.count;
+        const int *kinds = pl.d_kinds + ch.first;
+        hipLaunchKernelGGL(batched_reset_kernel, dim3(1), dim3(2), 0, s, pl.d_counter);
+        if (ch.general)
+            hipLaunchKernelGGL(batched_wave_kernel<false>, dim3(ch.general), dim3(64), wave::lds_bytes(pl.nmax), s, a,
+                               kinds);
+        if (ch.general < ch.count)
+            hipLaunchKernelGGL(batched_wave_kernel<true>, dim3(ch.count - ch.general), dim3(64),
+                               wave::lds_bytes(pl.nmax), s, a, kinds + ch.general);
+        // a persistent grid: one workgroup per CU (LDS allows one) pulls work from the queue
+        const int grid = std::min(ch.count, scirs::ctx().cu_count);
+        hipLaunchKernelGGL(batched_solve_kernel, dim3(grid), dim3(NT), 0, s, a);
+    }
     SCIRS_HIP_CHECK(hipGetLastError());
     return SCIRS_OK;
 }
@@ -554,6 +568,9 @@ extern "C" int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *n
     key = fnv1a(key, ptrs, sizeof(ptrs));
     key = fnv1a(key, &max_iter, sizeof(max_iter));
     key = fnv1a(key, &tol_scale, sizeof(tol_scale));
+    const char *wl = getenv("SCIRS_GPU_BATCH_WORK_MB");
+    const long limit = (wl && *wl && atol(wl) > 0 ? atol(wl) : BATCH_WORK_MB) * (1l << 17);   // doubles
+    key = fnv1a(key, &limit, sizeof(limit));
     const bool same = (pl.key == key && pl.batch == batch);
     if (!same) {
         pl.key = 0;       // no plan until this one is complete
@@ -564,17 +581,43 @@ extern "C" int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *n
         int nmax = 0;
         for (int i = 0; i < batch; ++i) {
             desc[i].n = n[i]; desc[i].nrhs = nrhs[i]; desc[i].spd = spd ? spd[i] : 0; desc[i].pad = 0;
-            desc[i].offA = offA[i]; desc[i].offB = offB[i]; desc[i].offW = work;
-            work += std::max(((long)n[i] * n[i] + 15) & ~15L, wave::work_doubles(n[i]));
+            desc[i].offA = offA[i]; desc[i].offB = offB[i];
             offP[i] = pw; pw += n[i];
             nmax = std::max(nmax, n[i]);
         }
         std::vector<int> order(batch);
         for (int i = 0; i < batch; ++i) order[i] = i;
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return n[x] > n[y]; });
-        std::vector<int> kinds(order);
-        pl.general = (int)(std::stable_partition(kinds.begin(), kinds.end(), [&](int x) { return !desc[x].spd; }) -
-                           kinds.begin());
+        std::vector<int> kinds;
+        // chunks of at most lim doubles of workspace
+        auto cut = [&](long lim) {
+            kinds = order;
+            pl.chunks.clear();
+            work = 0;
+            for (int first = 0; first < batch;) {
+                int last = first;
+                long used = 0;
+                for (; last < batch; ++last) {
+                    const int ni = n[order[last]];
+                    const long need = std::max(((long)ni * ni + 15) & ~15L, wave::work_doubles(ni));
+                    if (last > first && used + need > lim) break;
+                    desc[order[last]].offW = used;
+                    used += need;
+                }
+                work = std::max(work, used);
+                const auto k0 = kinds.begin() + first;
+                const auto mid = std::stable_partition(k0, kinds.begin() + last, [&](int x) { return !desc[x].spd; });
+                pl.chunks.push_back(BatchChunk{first, last - first, (int)(mid - k0)});
+                first = last;
+            }
+        };
+        // smaller chunks where memory is short
+        for (long lim = limit;; lim /= 4) {
+            cut(lim);
+            if (!(rc = grow(&pl.d_work, &pl.cap_work, (size_t)work))) break;
+            (void)hipGetLastError();
+            if (lim < (1l << 20)) return rc;
+        }
         if ((rc = grow(&pl.d_desc, &pl.cap_batch, batch))) return rc;
         size_t cap1 = 0, cap2 = 0, cap3 = 0, cap4 = 0, cap5 = 0, cap6 = 0;
         // the per-system arrays are (re)allocated together with the descriptors
@@ -585,7 +628,6 @@ extern "C" int scirs_gpu_dgesv_batched_dev(int batch, const int *n, const int *n
             (rc = grow(&pl.d_status, &cap4, batch)) || (rc = grow(&pl.d_iters, &cap5, batch)) ||
             (rc = grow(&pl.d_bwd, &cap6, batch)))
             return rc;
-        if ((rc = grow(&pl.d_work, &pl.cap_work, (size_t)work))) return rc;
         if ((rc = grow(&pl.d_perm, &pl.cap_perm, (size_t)pw))) return rc;
         if (!pl.d_counter) {
             size_t cc = 0;
