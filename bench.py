@@ -271,7 +271,7 @@ def bench_batched(args):
     t_loop = (time.perf_counter() - t0) / sample * args.batch
     roof_bw = bytes_alg / (info.time_ms * 1e-3) / 1e9
     line = {
-        "metric": "batched uneven solves/s (FP32 factor + FP64 refinement, one persistent launch)",
+        "metric": "batched uneven solves/s (FP32 factor + FP64 refinement, one call)",
         "value": args.batch / t,
         "unit": "solves/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": t * 1e3,

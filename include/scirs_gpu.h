@@ -242,7 +242,7 @@ int scirs_gpu_dgesv_ir_dev(int n, int nrhs, const double *dA, int64_t lda, const
  * (decomposition.rs:44, solve.rs:139) when spd[i] != 0 — computed as an FP32
  * factorisation plus FP64 refinement to a normwise backward error <= tol_scale *
  * n_i * 2^-53 (FP64 factorisation when FP32 breaks down or stalls), all systems in
- * one persistent, hipGraph-replayed launch.
+ * one replayed hipGraph: a launch per kind, one wave per system, and one for FP64.
  * Host arrays: n, nrhs (1 <= n <= 256, 1 <= nrhs <= 16), spd (may be NULL), offA,
  * offB (element offsets of A_i, row-major n_i x n_i, and of B_i / X_i, row-major
  * n_i x nrhs_i), status (out: 0, or the breakdown column / row), bwd (out, may be

@@ -19,7 +19,7 @@ struct Context {
     void *work_base = nullptr;
     void *host_flags = nullptr;
     int kb_f64 = 128, kb_f32 = 128, kb_chol = 128;
-    int narrow_kb = 1;   // narrower LU panels when a whole panel then fits one workgroup
+    int narrow_kb = 1;   // single 32-column LU sub-panels up to the rows where they win (scirs_lu_panel_kb)
     int chol_chain = 1;  // Cholesky solves through the chained triangular solve (else blocked)
     int trsv_dinv = 1;   // FP32 refinement solves with inverted 64 x 64 diagonal blocks
     // LU panel width for an m-row factorisation in element type T

@@ -16,7 +16,7 @@
 //     substitutions are then products only, for up to four right-hand sides at a time
 //   - residual rows come straight from A, 64 bytes per lane
 // 20000 systems of n ~ U[8,256], half of them Cholesky, 1 or 4 right-hand sides (3.6 GB
-// of input): 8.2 ms (general 4.8, SPD 3.4); 99.6 ms with a 256-thread workgroup per system,
+// of input): 8.1 ms (general 4.7, SPD 3.4); 99.6 ms with a 256-thread workgroup per system,
 // columns in LDS and substitutions in vector arithmetic.  What is left is HBM traffic: with
 // 2048 systems under way nothing stays in L2, A is read once to convert it and once per
 // refinement step, and the general systems moved 24.7 GB (4.2 TB/s; a copy reaches 4.8)
